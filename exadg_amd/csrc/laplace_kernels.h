@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "topology.h"
 
@@ -25,26 +26,31 @@ enum class ApplyMode : int
 };
 
 // Centrosymmetric n x n matrices (A_ij = A_{n-1-i,n-1-j}, such as the 1D mass and stiffness
-// on symmetric nodes) are stored for n >= 5 in even-odd form, which needs ~n^2/2 products per
+// on symmetric nodes) are stored in even-odd form, which needs ~n^2/2 products per
 // application instead of n^2: with m = n/2 and m_e = m + n%2,
 //   Ae (m x m_e): (A_ij + A_{i,n-1-j})/2 for j < m, A_im for j = m (odd n),
 //   Ao (m x m):   (A_ij - A_{i,n-1-j})/2,
 //   Am (m_e, odd n only): the middle row A_mj, j <= m.
-// The Cartesian kernel packs for n >= 5; the general kernel for n >= 6 (at n = 5 its saving
+// The Cartesian kernel packs at every n (its line Laplacian shares the even and odd parts with the
+// end derivatives and the flux terms); the general kernel for n >= 6 (at n = 5 its saving
 // is 4% of the instructions and the FP32 instantiation measured slower with it).
 constexpr int  eo_size(int n, bool packed)
 {
   return packed ? (n / 2) * (n / 2 + n % 2) + (n / 2) * (n / 2) + (n % 2 ? n / 2 + 1 : 0) : n * n;
 }
-constexpr bool cs_packed(int n) { return n >= 5; }
-constexpr int  cs_size(int n) { return eo_size(n, cs_packed(n)); }
+constexpr int  cs_size(int n) { return eo_size(n, true); }
 constexpr bool gen_packed(int n) { return n >= 6; }
 constexpr int  gen_size(int n) { return eo_size(n, gen_packed(n)); }
-// Offsets in the Cartesian kernel's table: [M | K | d0 n | d1 n], M and K of cs_size(n) each
+// Offsets in the Cartesian kernel's table: the unit-interval mass M in even-odd form, the end
+// derivative d0, d0 in even-odd form (DE_j = (d0_j + d0_{n-1-j})/2 for j < n/2 and d0_m in the
+// middle for odd n, DO_j = (d0_j - d0_{n-1-j})/2; the other end mirrors it, d1_j = -d0_{n-1-j}),
+// then per direction the stiffness times c/h and DE, DO times c/(2h), c the scale of the
+// direction's Kronecker term
 template<int N>
 struct CartTable
 {
-  static constexpr int M = 0, K = cs_size(N), D0 = 2 * cs_size(N), D1 = D0 + N;
+  static constexpr int M = 0, D0 = cs_size(N), DE = D0 + N, DO = DE + N / 2 + N % 2, L = D0 + 2 * N;
+  static constexpr int line(int d) { return L + d * (cs_size(N) + N); }
 };
 
 // Table layout (Number, SipgArgs::tab): general kernel: [S n*n | Dq n*n | d0 n | d1 n], and in
@@ -68,9 +74,10 @@ struct SipgArgs
   // kernel-argument loads (unit-interval mass M, stiffness K, end derivatives d0, d1, scaled
   // per direction inside the kernel); the general kernel (S, Dq, d0, d1) indexes them at run
   // time and reads the device copy `tables`.
-  static constexpr int kMaxTable = 2 * 9 * 9 + 2 * 9;
+  static constexpr int kMaxTable = 4 * cs_size(9) + 5 * 9;
   Number         tab[kMaxTable];
-  Number         h[6];  // Cartesian kernel: h_x, h_y, h_z, 1/h_x, 1/h_y, 1/h_z
+  // Cartesian kernel: the scales c_x = h_y h_z, ... of the three Kronecker terms, and c_d/(2 h_d)
+  Number         scale[3], half[3];
   Number const * tables;  // general kernel: the same tables in device memory
   Number const * src;
   Number *       dst;
@@ -85,6 +92,12 @@ struct SipgArgs
   // dst[(cell n^3 + probe) n^3 + e] (the block is symmetric, so this is also row `probe`)
   int            block = 0;
   int            tile_rows;  // traversal: y-rows per tile (one tile per XCD)
+  // Cartesian layered kernel: the penalty of a cell inside the mesh and what each boundary face
+  // normal to a direction adds; the lane assignment (cartesian_line_map, device memory) and the
+  // tiling, set by the launch
+  double         tau_base, tau_step[3];
+  int const *    line_map = nullptr;
+  int            row_length = 0, tiles = 0, layers_per_segment = 0;
   // chebyshev and residual modes
   Number const * x_old   = nullptr;
   Number const * rhs     = nullptr;
@@ -121,6 +134,12 @@ hipError_t launch_cartesian_diagonal(Number * diag, double const * diag1d, Numbe
 template<typename Number>
 hipError_t launch_general_diagonal(Number * diag, double const * tab1d, SipgArgs<Number> const & a,
                                    int degree, hipStream_t stream);
+
+// The lane assignment of the layered Cartesian kernel's x- and y-lines: per direction one entry per
+// lane, its LDS base | line << 16 (the two other coordinates, lower fastest) | the cell's column
+// and row in the tile << 23 and << 26, or -1; empty for degrees without that kernel
+template<typename Number>
+std::vector<int> cartesian_line_map(int degree);
 
 template<typename Number>
 hipError_t launch_sipg_cartesian(int degree, ApplyMode mode, SipgArgs<Number> const & args,

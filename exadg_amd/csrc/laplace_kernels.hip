@@ -1,6 +1,7 @@
-// SIPG Laplace operator kernels for CDNA4 (gfx950).
+// SIPG Laplace operator kernels for CDNA4 (gfx950): curved meshes, and the diagonals (the affine
+// operator is in cartesian_kernels.hip).
 //
-// Both kernels are element-centric: one group of (k+1)^2 lanes owns one cell, computes the
+// The operator kernels are element-centric: one group of (k+1)^2 lanes owns one cell, computes the
 // cell integral and all six face integrals seen from that cell (reading the neighbour's
 // lines from global memory / L2), and writes each dst entry exactly once -- no atomics.
 // A workgroup packs floor(256/(k+1)^2) cells; each cell gets its own LDS slice.
@@ -15,132 +16,13 @@
 
 #include "../../include/exadg_amd.h"
 #include "laplace_kernels.h"
+#include "sipg_lines.h"
 
 namespace ExaDG
 {
 namespace
 {
-constexpr int kInterior = 2;  // face type besides EXADG_BC_DIRICHLET / EXADG_BC_NEUMANN
-
 constexpr int cells_per_block(int n) { return (256 / (n * n)) > 0 ? 256 / (n * n) : 1; }
-
-// ---------------------------------------------------------------- line helpers
-
-// out[i] = sum_j M[i*N+j] in[j]
-template<int N, typename Number>
-__device__ __forceinline__ void mat_apply(Number const * __restrict__ M, Number const (&in)[N],
-                                          Number (&out)[N])
-{
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-  {
-    Number s = 0;
-#pragma unroll
-    for(int j = 0; j < N; ++j)
-      s += M[i * N + j] * in[j];
-    out[i] = s;
-  }
-}
-
-// out = A in for a centrosymmetric (Skew = false) or skew-centrosymmetric (Skew = true) A,
-// stored in even-odd form when Packed (see cs_packed / gen_packed), else as the plain row-major
-// matrix. Centro: out_i = E_i + O_i, out_{n-1-i} = E_i - O_i, middle output (odd n) from the
-// even part; skew: out_{n-1-i} = O_i - E_i and the middle output from the odd part.
-template<int N, bool Packed, bool Skew, typename Number>
-__device__ __forceinline__ void eo_apply(Number const * __restrict__ T, Number const (&in)[N],
-                                         Number (&out)[N])
-{
-  if constexpr(!Packed)
-    mat_apply<N>(T, in, out);
-  else
-  {
-    constexpr int  m = N / 2, me = m + N % 2;
-    Number const * Ae = T;
-    Number const * Ao = T + m * me;
-    Number const * Am = Ao + m * m;
-    Number         e[me], o[m];
-#pragma unroll
-    for(int j = 0; j < m; ++j)
-    {
-      e[j] = in[j] + in[N - 1 - j];
-      o[j] = in[j] - in[N - 1 - j];
-    }
-    if constexpr(N % 2 == 1)
-      e[m] = in[m];
-#pragma unroll
-    for(int i = 0; i < m; ++i)
-    {
-      Number E = 0, O = 0;
-#pragma unroll
-      for(int j = 0; j < me; ++j)
-        E += Ae[i * me + j] * e[j];
-#pragma unroll
-      for(int j = 0; j < m; ++j)
-        O += Ao[i * m + j] * o[j];
-      out[i]         = E + O;
-      out[N - 1 - i] = Skew ? O - E : E - O;
-    }
-    if constexpr(N % 2 == 1)
-    {
-      Number s = 0;
-      if constexpr(Skew)
-      {
-#pragma unroll
-        for(int j = 0; j < m; ++j)
-          s += Am[j] * o[j];
-      }
-      else
-      {
-#pragma unroll
-        for(int j = 0; j < me; ++j)
-          s += Am[j] * e[j];
-      }
-      out[m] = s;
-    }
-  }
-}
-
-// the Cartesian kernel's centrosymmetric 1D products (CartTable)
-template<int N, typename Number>
-__device__ __forceinline__ void cs_apply(Number const * __restrict__ T, Number const (&in)[N],
-                                         Number (&out)[N])
-{
-  eo_apply<N, cs_packed(N), false>(T, in, out);
-}
-
-// the general kernel's sweeps (GenTable): S and S^T centrosymmetric, Dq and Dq^T skew
-template<int N, bool Skew, typename Number>
-__device__ __forceinline__ void gen_apply(Number const * __restrict__ T, Number const (&in)[N],
-                                          Number (&out)[N])
-{
-  eo_apply<N, gen_packed(N), Skew>(T, in, out);
-}
-
-template<int N, typename Number>
-__device__ __forceinline__ void load_line(Number const * p, int stride, Number (&v)[N])
-{
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-    v[i] = p[i * stride];
-}
-
-template<int N, typename Number>
-__device__ __forceinline__ void store_line(Number * p, int stride, Number const (&v)[N])
-{
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-    p[i * stride] = v[i];
-}
-
-template<int N, typename Number>
-__device__ __forceinline__ Number dot_line(Number const * __restrict__ a, Number const (&v)[N])
-{
-  Number s = 0;
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-    s += a[i] * v[i];
-  return s;
-}
 
 // Base offset and stride of the line along direction d through lane (p,q) of an N^3 block;
 // (p,q) index the two other directions in increasing order.
@@ -162,18 +44,6 @@ __device__ __forceinline__ void line_geometry(int d, int p, int q, int & base, i
     base   = p + N * q;
     stride = N * N;
   }
-}
-
-// A store of an output that no kernel of the same apply reads back: marked non-temporal, so
-// that it does not displace from the caches the neighbour cells that other workgroups are
-// still reading. Used for the Cartesian vmult (FP64 k = 4: 7% faster on 64^3 cells, 3.5% on
-// 32^3; FP32 unchanged). The Chebyshev and residual outputs are read by the next kernel of a
-// V-cycle and stay cached (non-temporal there: V-cycle 0.8% slower), and the general kernel
-// keeps plain stores (0-3% slower with these).
-template<typename Number>
-__device__ __forceinline__ void store_stream(Number * p, Number v)
-{
-  __builtin_nontemporal_store(v, p);
 }
 
 // the cell's unit vector in diagonal (probing) mode, else the src line
@@ -736,383 +606,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// ================================================================ Cartesian kernel
-//
-// On an affine axis-parallel mesh the SIPG operator is exactly a sum of Kronecker products:
-//   A = L_x (x) M_y (x) M_z + M_x (x) L_y (x) M_z + M_x (x) M_y (x) L_z
-// with M_d = h_d * M (1D mass, exact with QGauss(k+1)) and L_d the 1D DG Laplacian along d:
-// K/h_d plus, at each line end, the flux terms of laplace_operator.h:180-197 written with
-// the exterior trace (value w and d/dx_d derivative dw at the shared face):
-//   right end: o_i -= 1/2 d1_i [u], o_{n-1} += -1/2 (du + dw) + tau [u],  [u] = u_{n-1} - w
-//   left end : o_i += 1/2 d0_i [u], o_0     +=  1/2 (du + dw) + tau [u],  [u] = u_0 - w
-// For boundary faces (w, dw) come from the mirror principle (weak_boundary_conditions.h):
-// Dirichlet w = -u, dw = du; Neumann w = u, dw = -du -- one branch-free code path.
-// Evaluated as out = M_z (M_y a_x + M_x a_y) + M_y M_x a_z with a_d = L_d(u, traces) in four
-// LDS phases (five workgroup barriers): the three a_d from x-, y- and z-lines; M_x a_y, M_x a_z
-// (x-lines) and M_y a_x (y-lines); M_y M_x a_z (y-lines) and M_z (...) (z-lines); the sum along
-// the z-lines. The neighbour lines are read once, at kernel start, and reduced to their traces.
-
-// LDS strides (x, y, z, cell) per n. n = 4 and 7 are padded to spread the 8-byte line
-// accesses of the three sweep orientations over the LDS banks; at n = 6 and 8 padding costs a
-// workgroup per CU in FP64 (measured 6-10% slower), so those are dense.
-template<int N>
-struct LdsLayout
-{
-  static constexpr int PX = N;
-  static constexpr int PY = (N == 4) ? 19 : (N == 7) ? 52 : N * N;
-  static constexpr int PC = (N == 4) ? 80 : (N == 7) ? 369 : N * N * N;
-};
-
-// a = c L_d u along one line: tab holds the unit-interval K, d0, d1; hinv = c/h_d and tau the
-// penalties times c, c being the scale of the Kronecker term. The neighbour derivative traces
-// dwnb are unit-interval derivatives as well (same h_d on a uniform box).
-template<int N, typename Number>
-__device__ __forceinline__ void line_laplacian(Number const * __restrict__ tab, Number hinv,
-                                               Number const (&u)[N], Number (&o)[N],
-                                               int const (&type)[2], Number const (&tau)[2],
-                                               Number const (&wnb)[2], Number const (&dwnb)[2])
-{
-  Number const * K  = tab + CartTable<N>::K;
-  Number const * d0 = tab + CartTable<N>::D0;
-  Number const * d1 = tab + CartTable<N>::D1;
-  cs_apply<N>(K, u, o);
-  Number const du0 = dot_line<N>(d0, u), du1 = dot_line<N>(d1, u);
-  // exterior traces: neighbour values or mirror values
-  Number const sl  = type[0] == EXADG_BC_DIRICHLET ? Number(-1) : Number(1);
-  Number const sr  = type[1] == EXADG_BC_DIRICHLET ? Number(-1) : Number(1);
-  Number const wl  = type[0] == kInterior ? wnb[0] : sl * u[0];
-  Number const dwl = type[0] == kInterior ? dwnb[0] : -sl * du0;
-  Number const wr  = type[1] == kInterior ? wnb[1] : sr * u[N - 1];
-  Number const dwr = type[1] == kInterior ? dwnb[1] : -sr * du1;
-  Number const jl = Number(0.5) * (u[0] - wl), jr = Number(0.5) * (u[N - 1] - wr);
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-    o[i] = hinv * (o[i] + d0[i] * jl - d1[i] * jr);
-  o[0] += hinv * Number(0.5) * (du0 + dwl) + Number(2) * tau[0] * jl;
-  o[N - 1] += Number(2) * tau[1] * jr - hinv * Number(0.5) * (du1 + dwr);
-}
-
-template<int N, typename Number, ApplyMode mode>
-__global__ void __launch_bounds__(256) sipg_cartesian_kernel(SipgArgs<Number> a)
-{
-  constexpr int N2 = N * N, N3 = N * N * N;
-  constexpr int CPB = cells_per_block(N);
-  using L           = LdsLayout<N>;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  Number *      smem   = reinterpret_cast<Number *>(smem_raw);
-  int const     slot   = threadIdx.x / N2;
-  int const     lt     = threadIdx.x - slot * N2;
-  int const     pos0   = (int)xcd_logical_block(blockIdx.x, gridDim.x) * CPB;
-  bool const    active = slot < CPB && pos0 + slot < (int)a.n_cells;
-  // three LDS buffers per cell: U (the cell's values), A and B; before the X phase A and B
-  // stage the two y-neighbour cells
-  Number *      U      = smem + (active ? slot : 0) * 3 * L::PC;
-  Number *      Abuf   = U + L::PC;
-  Number *      Bbuf   = Abuf + L::PC;
-  int const     p = lt % N, q = lt / N;
-  // LDS line bases of this lane for the x, y and z sweeps
-  int const     bx = L::PX * p + L::PY * q, by = p + L::PY * q, bz = p + L::PX * q;
-
-  int    type[3][2];
-  Number tau[3][2], wnb[3][2], dwnb[3][2];
-  Number own[N];  // this lane's z-line of the cell (lt + m N2), used by the Z phase
-  int    cell       = 0;
-  bool   in_block_l = false, in_block_r = false;
-  if(active)
-  {
-    int cc[3];
-    traversal_coords(a.topo, a.tile_rows, pos0, slot, cc);
-    int const nx = a.topo.nc[0], ny = a.topo.nc[1];
-    int const stride_c[3] = {1, nx, nx * ny};
-    cell                  = cc[0] + nx * (cc[1] + ny * cc[2]);
-    int nb[3][2];
-#pragma unroll
-    for(int d = 0; d < 3; ++d)
-    {
-      int const n_d = a.topo.nc[d], per = a.topo.periodic[d];
-      int const t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-      int const fbase =
-        (int)a.topo.face_base[d] + a.topo.layers[d] * (cc[t1] + a.topo.nc[t1] * cc[t2]);
-      nb[d][0] = cc[d] > 0 ? cell - stride_c[d] : (per ? cell + (n_d - 1) * stride_c[d] : -1);
-      nb[d][1] = cc[d] < n_d - 1 ? cell + stride_c[d] : (per ? cell - (n_d - 1) * stride_c[d] : -1);
-      int const fr = (per && cc[d] + 1 == n_d) ? 0 : cc[d] + 1;
-      tau[d][0]    = a.tau_face[fbase + cc[d]];
-      tau[d][1]    = a.tau_face[fbase + fr];
-#pragma unroll
-      for(int s = 0; s < 2; ++s)
-        type[d][s] = nb[d][s] >= 0 ? kInterior : a.topo.bc[2 * d + s];
-    }
-    if constexpr(mode == ApplyMode::diagonal)
-    {
-#pragma unroll
-      for(int m = 0; m < N; ++m)
-      {
-        own[m]            = (lt + m * N2 == a.probe) ? Number(1) : Number(0);
-        U[bz + L::PY * m] = own[m];
-      }
-      // neighbours contribute zero, except a cell that is its own periodic neighbour
-#pragma unroll
-      for(int d = 0; d < 3; ++d)
-      {
-        Number const * tb = a.tab;
-        int const      gbase = d == 0 ? N * (p + N * q) : d == 1 ? p + N2 * q : p + N * q;
-        int const      gstr  = d == 0 ? 1 : d == 1 ? N : N2;
-        Number         w[N];
-#pragma unroll
-        for(int i = 0; i < N; ++i)
-          w[i] = (gbase + i * gstr == a.probe) ? Number(1) : Number(0);
-        bool const self = nb[d][0] == cell;
-        wnb[d][0]       = self ? w[N - 1] : Number(0);
-        dwnb[d][0]      = self ? dot_line<N>(tb + CartTable<N>::D1, w) : Number(0);
-        wnb[d][1]       = self ? w[0] : Number(0);
-        dwnb[d][1]      = self ? dot_line<N>(tb + CartTable<N>::D0, w) : Number(0);
-      }
-    }
-    else
-    {
-      // All global loads up front. The own cell and the z- and y-neighbour cells are read in
-      // the same pattern (lane lt reads DoFs lt + m N^2: consecutive lanes, consecutive
-      // addresses); a lane then holds z-lines, so the z traces are lane-local and the
-      // y-neighbour cells go through LDS (A, B) to be read as y-lines. Only x-neighbours at
-      // the workgroup's ends are read as strided x-lines; the others come from U.
-      Number const * own_p = a.src + (size_t)cell * N3 + lt;
-      in_block_l = slot > 0 && cc[0] > 0;
-      in_block_r = slot + 1 < CPB && cc[0] + 1 < a.topo.nc[0] && pos0 + slot + 1 < (int)a.n_cells;
-      Number zl[N], zr[N], yl[N], yr[N], xl[N], xr[N];
-      Number const * pz0 = a.src + (size_t)(nb[2][0] >= 0 ? nb[2][0] : cell) * N3 + lt;
-      Number const * pz1 = a.src + (size_t)(nb[2][1] >= 0 ? nb[2][1] : cell) * N3 + lt;
-      Number const * py0 = a.src + (size_t)(nb[1][0] >= 0 ? nb[1][0] : cell) * N3 + lt;
-      Number const * py1 = a.src + (size_t)(nb[1][1] >= 0 ? nb[1][1] : cell) * N3 + lt;
-#pragma unroll
-      for(int m = 0; m < N; ++m)
-      {
-        own[m] = own_p[m * N2];
-        zl[m]  = pz0[m * N2];
-        zr[m]  = pz1[m * N2];
-        yl[m]  = py0[m * N2];
-        yr[m]  = py1[m * N2];
-      }
-      int const xbase = N * (p + N * q);  // this lane's x-line (y = p, z = q)
-      {
-        Number const * px0 = a.src + (size_t)(nb[0][0] >= 0 ? nb[0][0] : cell) * N3 + xbase;
-        Number const * px1 = a.src + (size_t)(nb[0][1] >= 0 ? nb[0][1] : cell) * N3 + xbase;
-#pragma unroll
-        for(int i = 0; i < N; ++i)
-        {
-          xl[i] = in_block_l ? Number(0) : px0[i];
-          xr[i] = in_block_r ? Number(0) : px1[i];
-        }
-      }
-#pragma unroll
-      for(int m = 0; m < N; ++m)
-      {
-        U[bz + L::PY * m]    = own[m];
-        Abuf[bz + L::PY * m] = yl[m];
-        Bbuf[bz + L::PY * m] = yr[m];
-      }
-      // lane-local traces (x ones are replaced from LDS for in-block neighbours)
-      Number const * tzb = a.tab;
-      Number const * txb = a.tab;
-      wnb[2][0]          = zl[N - 1];
-      dwnb[2][0]         = dot_line<N>(tzb + CartTable<N>::D1, zl);
-      wnb[2][1]          = zr[0];
-      dwnb[2][1]         = dot_line<N>(tzb + CartTable<N>::D0, zr);
-      wnb[0][0]          = xl[N - 1];
-      dwnb[0][0]         = dot_line<N>(txb + CartTable<N>::D1, xl);
-      wnb[0][1]          = xr[0];
-      dwnb[0][1]         = dot_line<N>(txb + CartTable<N>::D0, xr);
-    }
-  }
-  __syncthreads();
-  Number const * tx = a.tab;  // the same unit-interval tables in every direction
-  Number const * ty = a.tab;
-  Number const * tz = a.tab;
-  Number const   hx = a.h[0], hy = a.h[1], hz = a.h[2];
-  Number const   hxi = a.h[3], hyi = a.h[4], hzi = a.h[5];
-
-  // Scale factors of the three Kronecker terms: with M_d = h_d M (unit-interval mass M),
-  //   out = M_z M_y (c_x L_x u) + M_z M_x (c_y L_y u) + M_y M_x (c_z L_z u),
-  // c_x = h_y h_z, c_y = h_x h_z, c_z = h_x h_y, so that every mass sweep is a plain M.
-  Number const cx = hy * hz, cy = hx * hz, cz = hx * hy;
-  // P1: the remaining neighbour traces, then the three line Laplacians into registers
-  Number rx[N], ry[N], rz[N];
-  if(active)
-  {
-    if constexpr(mode != ApplyMode::diagonal)
-    {
-      // y traces from the staged neighbour cells, read as this lane's y-line (x = p, z = q)
-      Number w[N];
-      load_line<N>(Abuf + by, L::PX, w);
-      wnb[1][0]  = w[N - 1];
-      dwnb[1][0] = dot_line<N>(ty + CartTable<N>::D1, w);
-      load_line<N>(Bbuf + by, L::PX, w);
-      wnb[1][1]  = w[0];
-      dwnb[1][1] = dot_line<N>(ty + CartTable<N>::D0, w);
-      if(in_block_l)
-      {
-        load_line<N>(U - 3 * L::PC + bx, 1, w);
-        wnb[0][0]  = w[N - 1];
-        dwnb[0][0] = dot_line<N>(tx + CartTable<N>::D1, w);
-      }
-      if(in_block_r)
-      {
-        load_line<N>(U + 3 * L::PC + bx, 1, w);
-        wnb[0][1]  = w[0];
-        dwnb[0][1] = dot_line<N>(tx + CartTable<N>::D0, w);
-      }
-    }
-#pragma unroll
-    for(int d = 0; d < 3; ++d)
-    {
-      Number const c = d == 0 ? cx : d == 1 ? cy : cz;
-      tau[d][0] *= c;
-      tau[d][1] *= c;
-    }
-    Number u[N];
-    load_line<N>(U + bx, 1, u);
-    line_laplacian<N>(tx, cx * hxi, u, rx, type[0], tau[0], wnb[0], dwnb[0]);
-    load_line<N>(U + by, L::PX, u);
-    line_laplacian<N>(ty, cy * hyi, u, ry, type[1], tau[1], wnb[1], dwnb[1]);
-    line_laplacian<N>(tz, cz * hzi, own, rz, type[2], tau[2], wnb[2], dwnb[2]);
-  }
-  __syncthreads();  // U, A and B are read across lanes up to here
-  if(active)
-  {
-    store_line<N>(Abuf + bx, 1, rx);
-    store_line<N>(Bbuf + by, L::PX, ry);
-    store_line<N>(U + bz, L::PY, rz);
-  }
-  __syncthreads();
-  // P2: B <- M_x B and U <- M_x U along x-lines, A <- M_y A along y-lines (each line in place:
-  // in one phase every line of a buffer belongs to one lane)
-  if(active)
-  {
-    Number v[N], w[N];
-    load_line<N>(Bbuf + bx, 1, v);
-    cs_apply<N>(tx + CartTable<N>::M, v, w);
-    store_line<N>(Bbuf + bx, 1, w);
-    load_line<N>(U + bx, 1, v);
-    cs_apply<N>(tx + CartTable<N>::M, v, w);
-    store_line<N>(U + bx, 1, w);
-    load_line<N>(Abuf + by, L::PX, v);
-    cs_apply<N>(ty + CartTable<N>::M, v, w);
-    store_line<N>(Abuf + by, L::PX, w);
-  }
-  __syncthreads();
-  // P3: U <- M_y U along y-lines (the finished z-term); outp = M_z (A + B) along z-lines
-  Number outp[N];
-  if(active)
-  {
-    Number v[N], w[N];
-    load_line<N>(U + by, L::PX, v);
-    cs_apply<N>(ty + CartTable<N>::M, v, w);
-    store_line<N>(U + by, L::PX, w);
-    load_line<N>(Abuf + bz, L::PY, v);
-    load_line<N>(Bbuf + bz, L::PY, w);
-#pragma unroll
-    for(int i = 0; i < N; ++i)
-      v[i] += w[i];
-    cs_apply<N>(tz + CartTable<N>::M, v, outp);
-  }
-  __syncthreads();
-  if constexpr(mode == ApplyMode::residual_restrict)
-  {
-    // r = rhs - A u along the lane's z-line, restricted along z in registers, then along x and
-    // y through A and B (free after the barrier above); the coarse cell is added to dst
-    int const      nc = a.restrict_nc;
-    Number const * P  = a.restrict_P;  // P[i nc + c]: fine node i, coarse node c
-    if(active)
-    {
-      Number v[N], r[N];
-      load_line<N>(U + bz, L::PY, v);
-      size_t const g0 = (size_t)cell * N3 + lt;
-#pragma unroll
-      for(int k = 0; k < N; ++k)
-        r[k] = a.rhs[g0 + k * N2] - (outp[k] + v[k]);
-#pragma unroll
-      for(int c = 0; c < N; ++c)
-        if(c < nc)
-        {
-          Number s = 0;
-#pragma unroll
-          for(int k = 0; k < N; ++k)
-            s += P[k * nc + c] * r[k];
-          Abuf[p + N * q + N2 * c] = s;  // (x, y, c_z)
-        }
-    }
-    __syncthreads();
-    if(active && lt < N * nc)
-    {
-      int const y = lt % N, cz = lt / N;
-      for(int cx = 0; cx < nc; ++cx)
-      {
-        Number s = 0;
-#pragma unroll
-        for(int x = 0; x < N; ++x)
-          s += P[x * nc + cx] * Abuf[x + N * y + N2 * cz];
-        Bbuf[cx + nc * (y + N * cz)] = s;
-      }
-    }
-    __syncthreads();
-    if(active && lt < nc * nc)
-    {
-      int const     cx = lt % nc, cz = lt / nc;
-      int64_t const nc3 = (int64_t)nc * nc * nc;
-      for(int cy = 0; cy < nc; ++cy)
-      {
-        Number s = 0;
-#pragma unroll
-        for(int y = 0; y < N; ++y)
-          s += P[y * nc + cy] * Bbuf[cx + nc * (y + N * cz)];
-        a.dst[(int64_t)cell * nc3 + cx + nc * (cy + nc * cz)] += s;
-      }
-    }
-    return;
-  }
-  // out = outp + the z-term held in U, along the z-lines
-  if constexpr(mode == ApplyMode::diagonal)
-  {
-    if(active)
-    {
-      Number v[N];
-      load_line<N>(U + bz, L::PY, v);
-#pragma unroll
-      for(int k = 0; k < N; ++k)
-        if(a.block)
-          a.dst[((size_t)cell * N3 + a.probe) * N3 + lt + k * N2] = outp[k] + v[k];
-        else if(lt + k * N2 == a.probe)
-          a.dst[(size_t)cell * N3 + a.probe] = outp[k] + v[k];
-    }
-  }
-  else if(active)
-  {
-    // direct per-lane stores: lane (p, q) owns the z-line of DoFs lt + k N2 (a workgroup-wide
-    // LDS-staged store of the block's contiguous cells measured 10% slower)
-    Number v[N];
-    load_line<N>(U + bz, L::PY, v);
-    size_t const g0 = (size_t)cell * N3 + lt;
-#pragma unroll
-    for(int k = 0; k < N; ++k)
-    {
-      Number const ax = outp[k] + v[k];
-      size_t const g  = g0 + k * N2;
-      if constexpr(mode == ApplyMode::vmult)
-        store_stream(&a.dst[g], ax);
-      else if constexpr(mode == ApplyMode::vmult_add)
-        a.dst[g] += ax;
-      else if constexpr(mode == ApplyMode::residual)
-        a.dst[g] = a.rhs[g] - ax;
-      else
-      {
-        Number r = (Number(1) + a.f1) * own[k] + a.f2 * a.dinv[g] * (a.rhs[g] - ax);
-        if(a.has_old)
-          r -= a.f1 * a.x_old[g];
-        a.dst[g] = r;
-      }
-    }
-  }
-}
-
 template<int N, typename Number, ApplyMode mode>
 hipError_t launch_general_n(SipgArgs<Number> const & a, hipStream_t stream)
 {
@@ -1133,17 +626,6 @@ hipError_t launch_general_n(SipgArgs<Number> const & a, hipStream_t stream)
   return hipGetLastError();
 }
 
-template<int N, typename Number, ApplyMode mode>
-hipError_t launch_cartesian_n(SipgArgs<Number> const & a, hipStream_t stream)
-{
-  constexpr int CPB    = cells_per_block(N);
-  int const     blocks = (int)((a.n_cells + CPB - 1) / CPB);
-  size_t const  lds    = sizeof(Number) * CPB * 3 * LdsLayout<N>::PC;
-  hipLaunchKernelGGL((sipg_cartesian_kernel<N, Number, mode>), dim3(blocks), dim3(256), lds, stream,
-                     a);
-  return hipGetLastError();
-}
-
 template<typename Number, ApplyMode mode>
 hipError_t dispatch_general(int degree, SipgArgs<Number> const & a, hipStream_t s)
 {
@@ -1161,22 +643,6 @@ hipError_t dispatch_general(int degree, SipgArgs<Number> const & a, hipStream_t 
   }
 }
 
-template<typename Number, ApplyMode mode>
-hipError_t dispatch_cartesian(int degree, SipgArgs<Number> const & a, hipStream_t s)
-{
-  switch(degree)
-  {
-    case 1: return launch_cartesian_n<2, Number, mode>(a, s);
-    case 2: return launch_cartesian_n<3, Number, mode>(a, s);
-    case 3: return launch_cartesian_n<4, Number, mode>(a, s);
-    case 4: return launch_cartesian_n<5, Number, mode>(a, s);
-    case 5: return launch_cartesian_n<6, Number, mode>(a, s);
-    case 6: return launch_cartesian_n<7, Number, mode>(a, s);
-    case 7: return launch_cartesian_n<8, Number, mode>(a, s);
-    case 8: return launch_cartesian_n<9, Number, mode>(a, s);
-    default: return hipErrorInvalidValue;
-  }
-}
 // diagonal entry i of the 1D cell-local line operator along a direction of width h: the line
 // Laplacian of the Cartesian kernel applied to the unit vector e_i, with the exterior trace of
 // weak_boundary_conditions.h on boundary faces (type_l/type_r EXADG_BC_*), zero across interior
@@ -1454,26 +920,6 @@ hipError_t launch_sipg_general(int degree, ApplyMode mode, SipgArgs<Number> cons
 }
 
 template<typename Number>
-hipError_t launch_sipg_cartesian(int degree, ApplyMode mode, SipgArgs<Number> const & a,
-                                 hipStream_t s)
-{
-  switch(mode)
-  {
-    case ApplyMode::vmult: return dispatch_cartesian<Number, ApplyMode::vmult>(degree, a, s);
-    case ApplyMode::vmult_add: return dispatch_cartesian<Number, ApplyMode::vmult_add>(degree, a, s);
-    case ApplyMode::diagonal: return dispatch_cartesian<Number, ApplyMode::diagonal>(degree, a, s);
-    case ApplyMode::chebyshev:
-      return dispatch_cartesian<Number, ApplyMode::chebyshev>(degree, a, s);
-    case ApplyMode::residual: return dispatch_cartesian<Number, ApplyMode::residual>(degree, a, s);
-    case ApplyMode::residual_restrict:
-      if(a.restrict_P == nullptr || a.restrict_nc < 1 || a.restrict_nc > degree + 1)
-        return hipErrorInvalidValue;
-      return dispatch_cartesian<Number, ApplyMode::residual_restrict>(degree, a, s);
-  }
-  return hipErrorInvalidValue;
-}
-
-template<typename Number>
 hipError_t launch_cartesian_diagonal(Number * diag, double const * diag1d, Number const * tau_face,
                                      BoxTopology const & topo, double const (&h)[3], int n,
                                      int64_t n_cells, hipStream_t stream)
@@ -1517,7 +963,5 @@ template hipError_t launch_cartesian_diagonal<float>(float *, double const *, fl
                                                      int64_t, hipStream_t);
 template hipError_t launch_sipg_general<double>(int, ApplyMode, SipgArgs<double> const &, hipStream_t);
 template hipError_t launch_sipg_general<float>(int, ApplyMode, SipgArgs<float> const &, hipStream_t);
-template hipError_t launch_sipg_cartesian<double>(int, ApplyMode, SipgArgs<double> const &, hipStream_t);
-template hipError_t launch_sipg_cartesian<float>(int, ApplyMode, SipgArgs<float> const &, hipStream_t);
 
 }  // namespace ExaDG

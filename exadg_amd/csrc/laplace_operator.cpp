@@ -84,11 +84,39 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
   }
   else
   {
-    append(tab, even_odd_pack(shape_.mass, n, cs_packed(n), false));
-    append(tab, even_odd_pack(shape_.stiff, n, cs_packed(n), false));
+    // the end derivative d0 in even-odd form (CartTable); d1 mirrors it
+    int const           m = n / 2;
+    std::vector<double> de, scaled;
+    for(int j = 0; j < n; ++j)
+      if(std::abs(shape_.d1[j] + shape_.d0[n - 1 - j]) > 1e-12 * std::abs(shape_.d0[0]))
+        EXADG_THROW(EXADG_ERR_INTERNAL, "the 1D end derivatives do not mirror each other");
+    for(int j = 0; j < m; ++j)
+      de.push_back(0.5 * (shape_.d0[j] + shape_.d0[n - 1 - j]));
+    if(n % 2)
+      de.push_back(shape_.d0[m]);
+    for(int j = 0; j < m; ++j)
+      de.push_back(0.5 * (shape_.d0[j] - shape_.d0[n - 1 - j]));
+    append(tab, even_odd_pack(shape_.mass, n, true, false));
+    append(tab, shape_.d0);
+    append(tab, de);
+    for(int d = 0; d < 3; ++d)
+    {
+      double const c = grid_->h((d + 1) % 3) * grid_->h((d + 2) % 3), s = c / grid_->h(d);
+      scale_[d]      = (Number)c;
+      half_[d]       = (Number)(0.5 * s);
+      scaled         = even_odd_pack(shape_.stiff, n, true, false);
+      for(double & v : scaled)
+        v *= s;
+      append(tab, scaled);
+      scaled = de;
+      for(double & v : scaled)
+        v *= 0.5 * s;
+      append(tab, scaled);
+    }
+    std::vector<int> const map = cartesian_line_map<Number>(data.degree);
+    if(!map.empty())
+      line_map_.upload(map);
   }
-  append(tab, shape_.d0);
-  append(tab, shape_.d1);
   append(plain, curved ? shape_.S : shape_.mass);
   append(plain, curved ? shape_.Dq : shape_.stiff);
   append(plain, shape_.d0);
@@ -149,11 +177,6 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
     t[3 * n * n]     = shape_.d0[0];
     t[3 * n * n + 1] = shape_.d1[n - 1];
     diag_tab_.upload(t);
-  }
-  for(int d = 0; d < 3; ++d)
-  {
-    h_[d]     = (Number)grid_->h(d);
-    h_[3 + d] = (Number)(1.0 / grid_->h(d));
   }
   {
     // FP64 tables of the divergence right-hand side: S, Sd = Dq S, then weights and points
@@ -220,14 +243,23 @@ SipgArgs<Number> LaplaceOperator<Number>::make_args(Number * dst, Number const *
 {
   SipgArgs<Number> a;
   std::copy(tab_.begin(), tab_.end(), a.tab);
-  std::copy(h_, h_ + 6, a.h);
+  std::copy(scale_, scale_ + 3, a.scale);
+  std::copy(half_, half_ + 3, a.half);
   a.tables      = tables_.data();
   a.src         = src;
   a.dst         = dst;
   a.cell_metric = cell_metric_.data();
   a.face_data   = face_data_.data();
   a.tau_face    = tau_face_.data();
+  a.line_map    = line_map_.data();
   a.topo        = grid_->topology();
+  // tau_K = IP (k+1)^2 sum_f c_f |f| / |K| with c_f = 1/2 inside the mesh and 1 on its boundary
+  a.tau_base = 0;
+  for(int d = 0; d < 3; ++d)
+  {
+    a.tau_step[d] = 0.5 * data_.IP_factor * shape_.n * shape_.n / grid_->h(d);
+    a.tau_base += 2 * a.tau_step[d];
+  }
   a.n_cells     = grid_->n_cells();
   a.probe       = probe;
   // one tile of y-rows per XCD

@@ -174,8 +174,9 @@ private:
   GeometryData                          geo_;  // host copy (tau, and metric for curved)
   int                                   n3_;
   std::vector<Number>                   tab_;  // 1D tables (kernel-argument copy)
-  Number                                h_[6] = {1, 1, 1, 1, 1, 1};
+  Number                                scale_[3] = {1, 1, 1}, half_[3] = {1, 1, 1};
   DeviceBuffer<Number>                  tables_, cell_metric_, face_data_, tau_face_;
+  DeviceBuffer<int>                     line_map_;            // cartesian_line_map
   DeviceBuffer<double>                  diag1d_;              // affine: M_ii, K_ii, d0, d1 (FP64)
   DeviceBuffer<double>                  diag_tab_;            // curved: S^2, D^2, S D, l'(0), l'(1)
   DeviceBuffer<double>                  div_tables_;          // S, Sd, weights|points (FP64)

@@ -70,6 +70,37 @@ def test_vmult_fp64_matches_oracle(case, torch_cuda, product):
     assert _rel(ys.cpu().numpy(), 2 * y_ref) <= 1e-12
 
 
+# affine meshes just above the sizes where the layered kernel takes over (15 and 60 MB a vector in
+# FP32, 90 MB in FP64): rows that end inside a tile, odd last rows of tiles, segments of unequal
+# length, a box shorter than a tile, one layer, and every periodic direction
+LAYERED = [
+    (1, (79, 81, 75), "fp32", (0, 0, 0), (D, N, D, D, N, D)),
+    (1, (3, 7, 22500), "fp32", (0, 0, 0), (D,) * 6),
+    (1, (700, 680, 1), "fp32", (1, 1, 1), (D,) * 6),
+    (2, (53, 51, 53), "fp32", (1, 0, 0), (D, D, N, N, D, N)),
+    (3, (62, 61, 63), "fp32", (0, 1, 1), (N, D) * 3),
+    (4, (49, 51, 50), "fp32", (1, 1, 0), (N,) * 6),
+    (2, (76, 75, 74), "fp64", (0, 1, 0), (D, N, D, D, D, N)),
+    (3, (2, 89, 1000), "fp64", (1, 0, 1), (D, D, N, D, D, D)),
+]
+
+
+@pytest.mark.parametrize("k,nc,prec,per,bc", LAYERED, ids=[f"k{c[0]}-{c[2]}-{c[1]}" for c in LAYERED])
+def test_layered_vmult_matches_oracle(k, nc, prec, per, bc, torch_cuda, product):
+    torch = torch_cuda
+    case = ("layered", k, nc, 0.0, (1.0, 1.1, 0.9), 0.0, 1, 1, per, bc)
+    op_p, op_o = _build(product, case, product.FP32 if prec == "fp32" else product.FP64)
+    x = oracle.random_vector(op_o.n).astype(np.float32)
+    y_ref = op_o.vmult(x.astype(np.float64))
+    bar = 2e-6 if prec == "fp32" else 1e-12
+    xs = torch.from_numpy(x).cuda().to(op_p.dtype)
+    ys = torch.full_like(xs, float("nan"))
+    op_p.vmult(ys, xs)
+    assert _rel(ys.cpu().numpy(), y_ref) <= bar
+    op_p.vmult_add(ys, xs)
+    assert _rel(ys.cpu().numpy(), 2 * y_ref) <= bar
+
+
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}-k{c[1]}" for c in CASES])
 def test_vmult_fp32_matches_oracle(case, torch_cuda, product):
     """FP32 operator (the multigrid levels), vmult and vmult_add, on every mesh case."""
