@@ -384,6 +384,20 @@ bool Q1Operator<Number>::chebyshev_step(Number * x_new, Number const * x, Number
 }
 
 template<typename Number>
+bool Q1Operator<Number>::pcg(Q1PcgArgs<Number> args, hipStream_t s) const
+{
+  if(n_nodes_ > kQ1PcgMaxNodes)
+    return false;
+  args.W       = stencil_.data();
+  args.q       = q_;
+  args.n       = (int)n_nodes_;
+  hipError_t e = launch_q1_pcg<Number>(args, s);
+  if(e != hipSuccess)
+    EXADG_THROW(EXADG_ERR_HIP, hipGetErrorString(e));
+  return true;
+}
+
+template<typename Number>
 void Q1Operator<Number>::inverse_diagonal(Number * d, hipStream_t s) const
 {
   vec::copy(d, diag_.data(), n_nodes_, s);
@@ -1165,6 +1179,24 @@ void MultigridPreconditioner<Number>::coarse_solve(hipStream_t s)
   }
   // MGCoarseKrylov: r = src (mean removed if singular), PCG(Jacobi) from zero to
   // max(1e-12, rel_tol ||r0||)
+  Q1PcgArgs<Number> a;
+  a.x        = C.sol;
+  a.r        = cr_.data();
+  a.v        = coarse_ws_.v.data();
+  a.b        = C.defect.data();
+  a.dinv     = coarse_inv_diag_.data();
+  a.max_iter = data_.coarse_max_iter;
+  a.singular = data_.operator_is_singular;
+  a.rel_tol  = data_.coarse_rel_tol;
+  a.result   = red_.result();
+  if(C.op->pcg(a, s))
+  {
+    double const * h = red_.fetch(s, 2);
+    last_coarse_its_ = (int)h[0];
+    if(h[1] != 0.0)
+      EXADG_THROW(EXADG_ERR_NOT_FINITE, "non-finite residual in level CG");
+    return;
+  }
   vec::copy(cr_.data(), C.defect.data(), n, s);
   if(data_.operator_is_singular)
     vec::subtract_mean(red_, cr_.data(), n, s);

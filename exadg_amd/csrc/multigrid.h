@@ -193,6 +193,9 @@ public:
   {
     return false;
   }
+  // the coarse PCG solve in one launch (args without W, q and n); false if the level has no such form
+  // or is too large for it
+  virtual bool pcg(Q1PcgArgs<Number> /*args*/, hipStream_t /*s*/) const { return false; }
 };
 
 // continuous Q1 operator with strong Dirichlet constraints on the structured box
@@ -209,6 +212,7 @@ public:
   bool chebyshev_step(Number * x_new, Number const * x, Number const * x_old, Number const * b,
                       Number const * dinv, Number f1, Number f2, bool has_old,
                       hipStream_t s) const override;
+  bool pcg(Q1PcgArgs<Number> args, hipStream_t s) const override;
   Q1Topology const & q1_topology() const { return q_; }
   CGTopology const * cg_topology() const override { return &cg_; }
   std::vector<double> const & element_matrices() const { return mats_host_; }

@@ -72,6 +72,49 @@ def test_vcycle_fp64_matches_oracle(case, torch_cuda, product):
     assert err <= 1e-9
 
 
+# Q1 levels at the edges of the one-workgroup coarse PCG: nodes per thread 1 | 2 | more, its largest
+# level and the first one solved from the host; singular ones have their mean removed. The cells are
+# cubes: CG carries rounding of 1e-16 times the condition number of D^-1 A into its iterates, below
+# (136 nodes)^2 = 2e4 here, which stays under the bar by orders of magnitude (cells of aspect 340
+# instead reach 8e-8 at the same iterations)
+COARSE_PCG = [
+    # n_cells, periodic, bc, nodes
+    ((1, 1, 1), (0, 0, 0), (N,) * 5 + (D,), 8),
+    ((8, 8, 16), (1, 1, 1), (N,) * 6, 1024),
+    ((4, 4, 40), (0, 0, 0), (D,) * 5 + (N,), 1025),
+    ((8, 16, 16), (1, 1, 1), (N,) * 6, 2048),
+    ((40, 49, 1), (0, 0, 1), (D, N) * 3, 2050),
+    ((9, 9, 99), (0, 0, 0), (N,) * 5 + (D,), 10000),
+    ((72, 136, 1), (0, 0, 1), (D, N) * 3, 10001),
+]
+
+
+@pytest.mark.parametrize("nc,per,bc,nodes", COARSE_PCG, ids=[str(c[3]) for c in COARSE_PCG])
+def test_coarse_pcg_matches_oracle(nc, per, bc, nodes, torch_cuda, product):
+    """The V-cycle over DG 1 and the Q1 level solved by CG to 1e-3: the same iterations as the
+    oracle's, so the same V-cycle (FP64 1e-9, the bar above)."""
+    torch = torch_cuda
+    singular = D not in [b for d in range(3) if not per[d] for b in bc[2 * d:2 * d + 2]]
+    up = tuple(n / 10 for n in nc)
+    op = product.LaplaceOperator(product.mesh_desc(nc, 0.0, up, periodic=per), product.bc_desc(bc), 1)
+    prec = product.Preconditioner(op, product.PRECOND_MULTIGRID, product.mg_desc(
+        1, degrees=[1], precision=product.FP64, singular=singular))
+    mg_o = oracle.Multigrid(oracle.make_mesh(nc, 0.0, up, periodic=per, boundary_type=bc), [1],
+                            singular=singular)
+    assert prec.mg_levels()[0][3] == nodes == mg_o.sizes[0]
+    r = oracle.random_vector(op.n)
+    r -= r.mean() if singular else 0.0
+    z_ref = mg_o.vmult(r)
+    zs = torch.empty(op.n, dtype=torch.float64, device="cuda")
+    prec.vmult(zs, torch.from_numpy(r).cuda())
+    assert prec.mg_info()["last_coarse_iterations"] == mg_o.info().last_coarse_iterations
+    assert _rel(zs.cpu().numpy(), z_ref) <= 1e-9
+    r[1] = np.nan
+    with pytest.raises(product.ExaDGError) as e:
+        prec.vmult(zs, torch.from_numpy(r).cuda())
+    assert e.value.code == product.EXADG_ERR_NOT_FINITE
+
+
 @pytest.mark.parametrize("case", MG_CASES[:2], ids=[c[0] for c in MG_CASES[:2]])
 def test_vcycle_fp32_close_to_oracle(case, torch_cuda, product):
     torch = torch_cuda
