@@ -26,6 +26,21 @@ struct DivergenceArgs
 // velocity Neumann (u+ = u-: flux u-.n)
 hipError_t launch_divergence_apply(DivergenceArgs const & a, hipStream_t s);
 
+// The same on an affine box, without point data: G (n_p x n_u) = -int phi_i' psi_j and M = int phi_i
+// psi_j by the velocity quadrature on the unit interval, area the face areas per direction, which
+// the unit-interval masses of the other two directions complete to the cell.
+struct DivergenceAffineArgs
+{
+  double         G[81], M[81];
+  double         area[3];
+  double *       dst;
+  double const * src;
+  BoxTopology    topo;
+  int64_t        n_cells;
+};
+bool       has_divergence_affine(int n_u, int n_p);  // the pairs of sizes that have this kernel
+hipError_t launch_divergence_affine(DivergenceAffineArgs const & a, int n_u, int n_p, hipStream_t s);
+
 // u[c][k][node] = sum_m Re(d_m,k c_m exp(i 2 pi n_m.x_node)) at the given node positions
 // (3 x n_points, component-major); mode_data: 8 doubles per mode n(3), d(3), c_re, c_im,
 // |n_d| <= K <= 16. Nodes are numbered cell by cell (n3 per cell), the output in the velocity

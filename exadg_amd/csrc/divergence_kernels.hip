@@ -18,7 +18,7 @@ constexpr int kThreads = 256;
 // out[i + m0 (j + m1 k)] for in[a + n0 (b + n1 c)] with one matrix along one direction:
 // along direction `dir` apply M (rows: output index, m_out x m_in, M[o * m_in + a]), the
 // other two directions copied
-__device__ void sweep(double const * M, int m_out, int m_in, int dir, int const (&ext_in)[3],
+__device__ __forceinline__ void sweep(double const * M, int m_out, int m_in, int dir, int const (&ext_in)[3],
                       double const * in, double * out, bool transpose)
 {
   int ext_out[3] = {ext_in[0], ext_in[1], ext_in[2]};
@@ -39,10 +39,15 @@ __device__ void sweep(double const * M, int m_out, int m_in, int dir, int const 
   }
 }
 
+// NU, NP: nodes per direction of velocity and pressure, or 0 to take them from the arguments. With
+// the sizes known the index arithmetic of the sweeps (a dozen divisions per entry otherwise) folds
+// away.
+template<int NU, int NP>
 __global__ void __launch_bounds__(kThreads) divergence_apply_kernel(DivergenceArgs a)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  int const      nu = a.n_u, np = a.n_p, nu2 = nu * nu, nu3 = nu2 * nu, np3 = np * np * np;
+  int const      nu = NU ? NU : a.n_u, np = NP ? NP : a.n_p;
+  int const      nu2 = nu * nu, nu3 = nu2 * nu, np3 = np * np * np;
   double *       U   = reinterpret_cast<double *>(smem_raw);  // 3 nu^3 velocity, then Gauss data
   double *       T0  = U + 3 * nu3;                            // nu^3
   double *       T1  = T0 + nu3;                               // nu^3
@@ -196,6 +201,148 @@ __global__ void __launch_bounds__(kThreads) divergence_apply_kernel(DivergenceAr
     a.dst[c * np3 + e] = O[e];
 }
 
+// Affine boxes: the weak divergence is a sum of Kronecker products, one per velocity component,
+//   b = M_z M_y (G_x u_x) + M_x (M_z (G_y u_y) + M_y (G_z u_z)),
+// M_d = h_d M the rectangular mass matrix of pressure and velocity and G_d along the component's own
+// direction: -int phi_i' psi_j and the central flux at both ends, half of the own end value and
+// half of the neighbour's (all of the own one at an outflow, none at a wall). One group of n_u^2
+// lanes per cell, a line per lane; lines are contracted in place (a buffer line holds n_u or n_p
+// entries): G along x, y and z; M along y and z; M along z and x; the sum. No geometry is read.
+// Bound by HBM (the velocity in, the pressure out) and the LDS passes of the eight sweeps: k_u = 5,
+// k_p = 4 on 32^3 cells 56 us (3.7 TB/s of the 203 MB), the general kernel with its 0.9 GB of point
+// data 855 us.
+template<int NU, int NP>
+__global__ void __launch_bounds__(kThreads) divergence_affine_kernel(DivergenceAffineArgs a)
+{
+  constexpr int NU2 = NU * NU, NU3 = NU2 * NU, NP3 = NP * NP * NP;
+  constexpr int M  = NU > NP ? NU : NP;
+  constexpr int PY = M, PZ = M * M | 1, PC = PZ * (M - 1) + M * M;  // odd plane stride
+  constexpr int CPB = kThreads / NU2;
+  __shared__ double smem[CPB * 3 * PC];
+  int const         slot = threadIdx.x / NU2, lt = threadIdx.x - slot * NU2;
+  int64_t const     c      = xcd_logical_block(blockIdx.x, gridDim.x) * CPB + slot;
+  bool const        active = slot < CPB && c < a.n_cells;
+  double *          T[3];
+#pragma unroll
+  for(int k = 0; k < 3; ++k)
+    T[k] = smem + ((active ? slot : 0) * 3 + k) * PC;
+  double ends[3][2], we[3][2];  // neighbour's end value of this lane's line; weight of the own one
+  if(active)
+  {
+    double const * u = a.src + c * 3 * NU3;
+#pragma unroll
+    for(int k = 0; k < 3; ++k)
+#pragma unroll
+      for(int z = 0; z < NU; ++z)
+        T[k][lt % NU + PY * (lt / NU) + PZ * z] = u[k * NU3 + lt + NU2 * z];
+    int cc[3];
+    cell_coords(a.topo, c, cc);
+#pragma unroll
+    for(int d = 0; d < 3; ++d)
+#pragma unroll
+      for(int s = 0; s < 2; ++s)
+      {
+        int64_t const nb   = neighbor_id(a.topo, cc, d, s);
+        int const     p = lt % NU, q = lt / NU, end = s ? 0 : NU - 1;
+        int const     at = d == 0 ? end + NU * lt : d == 1 ? p + NU * end + NU2 * q : lt + NU2 * end;
+        ends[d][s] = nb >= 0 ? 0.5 * a.src[(nb * 3 + d) * NU3 + at] : 0.0;
+        we[d][s]   = nb >= 0 ? 0.5 : a.topo.bc[2 * d + s] == EXADG_BC_DIRICHLET ? 1.0 : 0.0;
+      }
+  }
+  __syncthreads();
+  if(active)
+  {
+    int const p = lt % NU, q = lt / NU;
+#pragma unroll
+    for(int d = 0; d < 3; ++d)
+    {
+      int const base = d == 0 ? PY * p + PZ * q : d == 1 ? p + PZ * q : p + PY * q;
+      int const st   = d == 0 ? 1 : d == 1 ? PY : PZ;
+      double    v[NU];
+#pragma unroll
+      for(int i = 0; i < NU; ++i)
+        v[i] = T[d][base + i * st];
+      double const lo = we[d][0] * v[0] + ends[d][0], up = we[d][1] * v[NU - 1] + ends[d][1];
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        double s = 0;
+#pragma unroll
+        for(int j = 0; j < NU; ++j)
+          s += a.G[i * NU + j] * v[j];
+        if(i == 0)
+          s -= lo;
+        if(i == NP - 1)
+          s += up;
+        T[d][base + i * st] = a.area[d] * s;
+      }
+    }
+  }
+  __syncthreads();
+  // T <- M T along one direction, for the lines of e0 x e1 entries of the two others
+  auto mass = [&](double const * in, double const * in2, double * out, int d, int e0, int e1) {
+    for(int t = lt; t < e0 * e1; t += NU2)
+    {
+      int const p = t % e0, q = t / e0;
+      int const base = d == 0 ? PY * p + PZ * q : d == 1 ? p + PZ * q : p + PY * q;
+      int const st   = d == 0 ? 1 : d == 1 ? PY : PZ;
+      double    v[NU];
+#pragma unroll
+      for(int i = 0; i < NU; ++i)
+        v[i] = in2 ? in[base + i * st] + in2[base + i * st] : in[base + i * st];
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        double s = 0;
+#pragma unroll
+        for(int j = 0; j < NU; ++j)
+          s += a.M[i * NU + j] * v[j];
+        out[base + i * st] = s;
+      }
+    }
+  };
+  if(active)
+  {
+    mass(T[0], nullptr, T[0], 1, NP, NU);  // (i0, z)
+    mass(T[2], nullptr, T[2], 1, NU, NP);  // (x, i2)
+    mass(T[1], nullptr, T[1], 2, NU, NP);  // (x, i1)
+  }
+  __syncthreads();
+  if(active)
+  {
+    mass(T[0], nullptr, T[0], 2, NP, NP);
+    mass(T[1], T[2], T[1], 0, NP, NP);
+  }
+  __syncthreads();
+  if(active)
+    for(int e = lt; e < NP3; e += NU2)
+    {
+      int const at          = e % NP + PY * (e / NP % NP) + PZ * (e / (NP * NP));
+      a.dst[c * NP3 + e] = T[0][at] + T[1][at];
+    }
+}
+
+template<int NU, int NP>
+hipError_t launch_affine(DivergenceAffineArgs const & a, hipStream_t s)
+{
+  constexpr int CPB = kThreads / (NU * NU);
+  hipLaunchKernelGGL((divergence_affine_kernel<NU, NP>), dim3((unsigned)((a.n_cells + CPB - 1) / CPB)),
+                     dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+template<int NU, int NP>
+hipError_t launch_general(DivergenceArgs const & a, hipStream_t s)
+{
+  int const    nu = a.n_u, np = a.n_p;
+  size_t const lds = sizeof(double) * (5 * nu * nu * nu + np * np * np + 13 * nu * nu);
+  if(lds > 65536)
+    return hipErrorInvalidValue;  // at most 5 * 729 + 729 + 1053 doubles = 43.6 KB for n <= 9
+  hipLaunchKernelGGL((divergence_apply_kernel<NU, NP>), dim3((unsigned)a.n_cells), dim3(kThreads), lds, s,
+                     a);
+  return hipGetLastError();
+}
+
 // one thread per node; per-thread tables e^{2 pi i m x_d}, m = 0..K, in LDS
 constexpr int kInterpThreads = 128;
 
@@ -252,11 +399,33 @@ hipError_t launch_divergence_apply(DivergenceArgs const & a, hipStream_t s)
   if(nu < 2 || nu > 9 || np < 2 || np > 9 || a.n_cells < 1 || !a.dst || !a.src || !a.cell_geo ||
      !a.face_geo || !a.tables)
     return hipErrorInvalidValue;
-  size_t const lds = sizeof(double) * (5 * nu * nu * nu + np * np * np + 13 * nu * nu);
-  if(lds > 65536)
-    return hipErrorInvalidValue;  // at most 5 * 729 + 729 + 1053 doubles = 43.6 KB for n <= 9
-  hipLaunchKernelGGL(divergence_apply_kernel, dim3((unsigned)a.n_cells), dim3(kThreads), lds, s, a);
-  return hipGetLastError();
+  // the pairs of degrees in use: velocity of one degree more than the pressure, or equal
+#define EXADG_CASE(NU, NP)      \
+  if(nu == NU && np == NP)      \
+    return launch_general<NU, NP>(a, s);
+  EXADG_CASE(3, 2) EXADG_CASE(4, 3) EXADG_CASE(5, 4) EXADG_CASE(6, 5) EXADG_CASE(7, 6) EXADG_CASE(8, 7)
+  EXADG_CASE(9, 8)
+  EXADG_CASE(2, 2) EXADG_CASE(3, 3) EXADG_CASE(4, 4) EXADG_CASE(5, 5) EXADG_CASE(6, 6) EXADG_CASE(7, 7)
+  EXADG_CASE(8, 8) EXADG_CASE(9, 9)
+#undef EXADG_CASE
+  return launch_general<0, 0>(a, s);
+}
+
+bool has_divergence_affine(int nu, int np) { return nu >= 2 && nu <= 9 && np >= 2 && (np == nu || np == nu - 1); }
+
+hipError_t launch_divergence_affine(DivergenceAffineArgs const & a, int nu, int np, hipStream_t s)
+{
+  if(!has_divergence_affine(nu, np) || a.n_cells < 1 || !a.dst || !a.src)
+    return hipErrorInvalidValue;
+#define EXADG_CASE(NU, NP)      \
+  if(nu == NU && np == NP)      \
+    return launch_affine<NU, NP>(a, s);
+  EXADG_CASE(3, 2) EXADG_CASE(4, 3) EXADG_CASE(5, 4) EXADG_CASE(6, 5) EXADG_CASE(7, 6) EXADG_CASE(8, 7)
+  EXADG_CASE(9, 8)
+  EXADG_CASE(2, 2) EXADG_CASE(3, 3) EXADG_CASE(4, 4) EXADG_CASE(5, 5) EXADG_CASE(6, 6) EXADG_CASE(7, 7)
+  EXADG_CASE(8, 8) EXADG_CASE(9, 9)
+#undef EXADG_CASE
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_fourier_interpolate(double * u, double const * x_nodes, double const * mode_data,

@@ -32,6 +32,27 @@ DivergenceOperator::DivergenceOperator(std::shared_ptr<StructuredGrid const> gri
   tab.insert(tab.end(), Sp.begin(), Sp.end());
   tab.insert(tab.end(), Sdp.begin(), Sdp.end());
   tables_.upload(tab);
+  affine_ = grid_->affine() && has_divergence_affine(nu, np);
+  if(affine_)
+  {
+    for(int i = 0; i < np; ++i)
+      for(int j = 0; j < nu; ++j)
+      {
+        double g = 0, m = 0;
+        for(int q = 0; q < nu; ++q)
+        {
+          g -= su.qw[q] * Sdp[q * np + i] * su.S[q * nu + j];
+          m += su.qw[q] * Sp[q * np + i] * su.S[q * nu + j];
+        }
+        affine_args_.G[i * nu + j] = g;
+        affine_args_.M[i * nu + j] = m;
+      }
+    for(int d = 0; d < 3; ++d)
+      affine_args_.area[d] = grid_->h((d + 1) % 3) * grid_->h((d + 2) % 3);
+    affine_args_.topo    = grid_->topology();
+    affine_args_.n_cells = grid_->n_cells();
+    return;  // no point data
+  }
   // point data at the velocity quadrature (positions, JxW J^{-1}; face JxW n)
   DivergenceGeometry const g = compute_divergence_geometry(*grid_, su);
   cell_geo_.upload(g.cell);
@@ -44,6 +65,16 @@ void DivergenceOperator::apply(double * dst, double const * src, hipStream_t s) 
     EXADG_THROW(EXADG_ERR_ARGUMENT, "null vector");
   if((void const *)dst == (void const *)src)
     EXADG_THROW(EXADG_ERR_ARGUMENT, "dst and src must not alias");
+  if(affine_)
+  {
+    DivergenceAffineArgs a = affine_args_;
+    a.dst                  = dst;
+    a.src                  = src;
+    hipError_t const e     = launch_divergence_affine(a, degree_u_ + 1, degree_p_ + 1, s);
+    if(e != hipSuccess)
+      EXADG_THROW(EXADG_ERR_HIP, std::string("divergence kernel launch: ") + hipGetErrorString(e));
+    return;
+  }
   DivergenceArgs a;
   a.dst      = dst;
   a.src      = src;

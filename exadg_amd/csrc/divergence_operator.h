@@ -38,6 +38,8 @@ private:
   std::shared_ptr<StructuredGrid const> grid_;
   int                                   degree_p_, degree_u_, nu3_, np3_;
   DeviceBuffer<double>                  tables_, cell_geo_, face_geo_;
+  bool                                  affine_ = false;  // the affine kernel, without point data
+  DivergenceAffineArgs                  affine_args_;
   mutable DeviceBuffer<double>          nodes_, modes_;
 };
 }  // namespace ExaDG

@@ -18,6 +18,14 @@ CASES = [
     ("curved_periodic", (2, 3, 2), 0.08, 4, (1, 0, 1), (D,) * 6, 4, 4),
     ("single_periodic", (1, 2, 2), 0.0, 1, (1, 0, 0), (N,) * 6, 1, 2),
     ("curved_k5", (2, 2, 2), 0.1, 5, (1, 1, 0), (N,) * 6, 5, 6),
+    # the affine kernel's other pairs of degrees (largest, smallest, equal), more cells than one
+    # workgroup holds, and a pair that only the general kernel has
+    ("cart_k8", (2, 3, 2), 0.0, 1, (0, 1, 0), (N, D, N, N, D, N), 7, 8),
+    ("cart_equal_k8", (2, 2, 2), 0.0, 1, (0, 0, 0), (D, N) * 3, 8, 8),
+    ("cart_equal_k1", (7, 5, 4), 0.0, 1, (0, 0, 1), (N, D) * 3, 1, 1),
+    ("cart_k6", (3, 2, 3), 0.0, 1, (0, 0, 0), (N,) * 6, 5, 6),
+    ("cart_general_pair", (3, 2, 2), 0.0, 1, (0, 1, 0), (N, D) * 3, 2, 5),
+    ("curved_equal_k8", (2, 2, 2), 0.1, 2, (1, 0, 0), (D,) * 6, 8, 8),
 ]
 
 
