@@ -100,34 +100,38 @@ void GuessNet::ensure_workspace(int B)
 float const * GuessNet::forward(float const * X, int B, hipStream_t s)
 {
   ensure_workspace(B);
-  int const w = width_;
-  check_launch(launch_sgemm(B, w, F_, X, F_, 1, W1(), 1, F_, H1_.data(), w, 1.f, false, b1(), true, nullptr, 0, s));
-  check_launch(launch_sgemm(B, w, w, H1_.data(), w, 1, W2(), 1, w, H2_.data(), w, 1.f, false, b2(), true, nullptr, 0, s));
-  check_launch(launch_sgemm(B, n3_, w, H2_.data(), w, 1, W3(), 1, w, Y_.data(), n3_, 1.f, false, b3(), false, nullptr, 0, s));
+  // H = act(in W^T + b), W row-major (out x in)
+  auto layer = [&](float const * in, int n_in, float const * W, float const * b, int n_out, float * out,
+                   bool relu) {
+    SgemmArgs a{B, n_out, n_in, in, n_in, 1, W, 1, n_in, out, n_out};
+    a.bias = b;
+    a.relu = relu;
+    check_launch(launch_sgemm(a, nullptr, 0, s));
+  };
+  layer(X, F_, W1(), b1(), width_, H1_.data(), true);
+  layer(H1_.data(), width_, W2(), b2(), width_, H2_.data(), true);
+  layer(H2_.data(), width_, W3(), b3(), n3_, Y_.data(), false);
   return Y_.data();
 }
 
 void GuessNet::backward(float const * X, int B, hipStream_t s)
 {
-  int const w = width_;
-  // output layer
-  check_launch(launch_sgemm(n3_, w, B, dY_.data(), 1, n3_, H2_.data(), w, 1, gW(W3()), w, 1.f, false, nullptr, false, split_.data(),
-                            (int64_t)split_.size(), s));
-  check_launch(launch_column_sum(dY_.data(), B, n3_, gW(b3()), s));
-  check_launch(launch_sgemm(B, w, n3_, dY_.data(), n3_, 1, W3(), w, 1, dH2_.data(), w, 1.f, false, nullptr, false, split_.data(),
-                            (int64_t)split_.size(), s));
-  check_launch(launch_relu_backward(dH2_.data(), H2_.data(), (int64_t)B * w, s));
-  // hidden layer 2
-  check_launch(launch_sgemm(w, w, B, dH2_.data(), 1, w, H1_.data(), w, 1, gW(W2()), w, 1.f, false, nullptr, false, split_.data(),
-                            (int64_t)split_.size(), s));
-  check_launch(launch_column_sum(dH2_.data(), B, w, gW(b2()), s));
-  check_launch(launch_sgemm(B, w, w, dH2_.data(), w, 1, W2(), w, 1, dH1_.data(), w, 1.f, false, nullptr, false, split_.data(),
-                            (int64_t)split_.size(), s));
-  check_launch(launch_relu_backward(dH1_.data(), H1_.data(), (int64_t)B * w, s));
-  // hidden layer 1
-  check_launch(launch_sgemm(w, F_, B, dH1_.data(), 1, w, X, F_, 1, gW(W1()), F_, 1.f, false, nullptr, false, split_.data(),
-                            (int64_t)split_.size(), s));
-  check_launch(launch_column_sum(dH1_.data(), B, w, gW(b1()), s));
+  // gradients of a layer's weights (dOut^T in) and biases (column sums of dOut, the row sums of the
+  // GEMM's A), and of its input (dOut W, zero where the ReLU before it was)
+  auto layer = [&](float const * d_out, int n_out, float const * in, int n_in, float * W,
+                   float * b, float * d_in) {
+    SgemmArgs w{n_out, n_in, B, d_out, 1, n_out, in, n_in, 1, gW(W), n_in};
+    w.row_sum = gW(b);
+    check_launch(launch_sgemm(w, split_.data(), (int64_t)split_.size(), s));
+    if(d_in == nullptr)
+      return;
+    SgemmArgs a{B, n_in, n_out, d_out, n_out, 1, W, n_in, 1, d_in, n_in};
+    a.mask = in;
+    check_launch(launch_sgemm(a, split_.data(), (int64_t)split_.size(), s));
+  };
+  layer(dY_.data(), n3_, H2_.data(), width_, W3(), b3(), dH2_.data());
+  layer(dH2_.data(), width_, H1_.data(), width_, W2(), b2(), dH1_.data());
+  layer(dH1_.data(), width_, X, F_, W1(), b1(), nullptr);
 }
 
 double GuessNet::loss_and_grad(float const * X, float const * T, int B, hipStream_t s)

@@ -24,13 +24,27 @@ struct FeatureScales
   float inv_t    = 1.f;
 };
 
-// C(i,j) = alpha sum_k A(i,k) B(k,j) (+ C) (+ bias_j) (ReLU), A(i,k) = A[i a_i + k a_k],
-// B(k,j) = B[k b_k + j b_j]; with a workspace of >= s*M*N floats the K range may be split
-// over s blocks when M x N alone has too few tiles
-hipError_t launch_sgemm(int M, int N, int K, float const * A, int64_t a_i, int64_t a_k,
-                        float const * B, int64_t b_k, int64_t b_j, float * C, int64_t ldc,
-                        float alpha, bool accumulate, float const * bias, bool relu,
-                        float * workspace, int64_t workspace_floats, hipStream_t s);
+// C(i,j) = alpha sum_k A(i,k) B(k,j) (+ C if accumulate) (+ bias_j) (ReLU) (0 where mask(i,j) <= 0,
+// laid out as C), A(i,k) = A[i a_i + k a_k], B(k,j) = B[k b_k + j b_j], one of the two strides of
+// each being 1; row_sum (if not null) receives sum_k A(i,k). With a workspace of >= s M (N + 1)
+// floats the K range may be split over s blocks when M x N alone has too few tiles.
+struct SgemmArgs
+{
+  int           M, N, K;
+  float const * A;
+  int64_t       a_i, a_k;
+  float const * B;
+  int64_t       b_k, b_j;
+  float *       C;
+  int64_t       ldc;
+  float         alpha      = 1.f;
+  int           accumulate = 0;
+  float const * bias       = nullptr;
+  int           relu       = 0;
+  float const * mask       = nullptr;
+  float *       row_sum    = nullptr;
+};
+hipError_t launch_sgemm(SgemmArgs const & a, float * workspace, int64_t workspace_floats, hipStream_t s);
 template<typename In>
 hipError_t launch_features(float * X, float * T, History<In> const & hist, In const * rhs,
                            In const * target, int history, int n_cell_dofs, int64_t cell0, int B,
@@ -42,8 +56,6 @@ hipError_t launch_feature_moments(float const * X, float const * T, int history,
 // dY = 2 scale (Y - T); loss_sum (+)= sum (Y - T)^2
 hipError_t launch_mse_backward(float const * Y, float const * T, float * dY, int64_t n, float scale,
                                double * partial, double * loss_sum, bool accumulate, hipStream_t s);
-hipError_t launch_relu_backward(float * dH, float const * H, int64_t n, hipStream_t s);
-hipError_t launch_column_sum(float const * dY, int M, int N, float * db, hipStream_t s);
 hipError_t launch_adam(float * p, float const * g, float * m, float * v, int64_t n, float lr,
                        float b1, float b2, float eps, int step, hipStream_t s);
 // x0 = sum_h beta_h hist_h (+ st * Y) (- target); counts the non-finite entries of Y into n_bad

@@ -1,6 +1,5 @@
-// Kernels of the learned initial guess (per-cell MLP, FP32): a tiled GEMM on the matrix cores
-// with strided operands, feature gathering from a solution history, ReLU and MSE backward,
-// bias gradients, Adam; plus the FP64 extrapolation of the initial guess
+// Kernels of the learned initial guess (per-cell MLP, FP32) besides its GEMM (sgemm_kernels.hip):
+// feature gathering from a solution history, MSE backward, Adam; plus the FP64 extrapolation of the initial guess
 // (time_integration/extrapolation_constants.cpp:55-93) and the right-hand side of the
 // pressure sequence: the weak DG divergence with central flux (divergence_operator.h:63-68,
 // divergence_operator.cpp:190-215) of an analytic Fourier velocity field.
@@ -14,123 +13,6 @@ namespace ExaDG
 {
 namespace
 {
-constexpr int TM = 64, TN = 64, TK = 16;
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// C(i,j) = alpha * sum_k A(i,k) B(k,j) (+ C) (+ bias_j), optional ReLU, on the matrix cores:
-// each of the 4 waves computes a 32 x 32 quadrant of the 64 x 64 tile as 2 x 2 products
-// v_mfma_f32_16x16x4f32 (FP32 operands, FP32 accumulation). Lane l supplies A(l%16, l/16) and
-// B(l/16, l%16) of a 16 x 4 / 4 x 16 step and holds D(4 (l/16) + r, l%16), r = 0..3.
-// A(i,k) = A[i*a_i + k*a_k], B(k,j) = B[k*b_k + j*b_j], C row-major with leading dim ldc.
-// With gridDim.z > 1 (split K), block z covers k in [z*kc, min(K, (z+1)*kc)) and writes its
-// raw partial product to C + z * M * ldc; splitk_reduce_kernel applies alpha/C/bias/ReLU.
-__global__ void __launch_bounds__(256)
-  sgemm_kernel(int M, int N, int K, float const * __restrict__ A, int64_t a_i, int64_t a_k,
-               float const * __restrict__ B, int64_t b_k, int64_t b_j, float * __restrict__ C,
-               int64_t ldc, float alpha, int accumulate, float const * __restrict__ bias, int relu,
-               int kc)
-{
-  __shared__ float As[TK][TM + 1];
-  __shared__ float Bs[TK][TN + 1];
-  int const tid = threadIdx.x;
-  int const i0 = blockIdx.y * TM, j0 = blockIdx.x * TN;
-  int const kb = blockIdx.z * kc, ke = min(K, kb + kc);
-  bool const split = gridDim.z > 1;
-  if(split)
-  {
-    C += (int64_t)blockIdx.z * M * ldc;
-    alpha = 1.f, accumulate = 0, bias = nullptr, relu = 0;
-  }
-  int const lane = tid & 63, wave = tid >> 6;
-  int const wr = 32 * (wave >> 1), wc = 32 * (wave & 1);  // this wave's quadrant
-  int const li = lane & 15, lk = lane >> 4;
-  f32x4     acc[2][2];
-#pragma unroll
-  for(int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for(int cb = 0; cb < 2; ++cb)
-      acc[rb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for(int k0 = kb; k0 < ke; k0 += TK)
-  {
-    // 64x16 tiles of A and 16x64 of B: 4 elements per thread each
-    for(int e = tid; e < TM * TK; e += 256)
-    {
-      int const r = e / TK, c = e % TK;
-      int const i = i0 + r, k = k0 + c;
-      As[c][r]    = (i < M && k < ke) ? A[i * a_i + k * a_k] : 0.f;
-    }
-    for(int e = tid; e < TK * TN; e += 256)
-    {
-      int const r = e / TN, c = e % TN;
-      int const k = k0 + r, j = j0 + c;
-      Bs[r][c]    = (k < ke && j < N) ? B[k * b_k + j * b_j] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for(int kk = 0; kk < TK; kk += 4)
-    {
-      float a[2], b[2];
-#pragma unroll
-      for(int rb = 0; rb < 2; ++rb)
-        a[rb] = As[kk + lk][wr + 16 * rb + li];
-#pragma unroll
-      for(int cb = 0; cb < 2; ++cb)
-        b[cb] = Bs[kk + lk][wc + 16 * cb + li];
-#pragma unroll
-      for(int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for(int cb = 0; cb < 2; ++cb)
-          acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rb], b[cb], acc[rb][cb], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for(int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for(int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for(int r = 0; r < 4; ++r)
-      {
-        int const i = i0 + wr + 16 * rb + 4 * lk + r;
-        int const j = j0 + wc + 16 * cb + li;
-        if(i >= M || j >= N)
-          continue;
-        float v = alpha * acc[rb][cb][r];
-        if(accumulate)
-          v += C[i * ldc + j];
-        if(bias)
-          v += bias[j];
-        if(relu)
-          v = v > 0.f ? v : 0.f;
-        C[i * ldc + j] = v;
-      }
-}
-
-__global__ void __launch_bounds__(256)
-  splitk_reduce_kernel(int M, int N, int splits, float const * __restrict__ part, float * C,
-                       int64_t ldc, float alpha, int accumulate, float const * __restrict__ bias,
-                       int relu)
-{
-  int64_t const total = (int64_t)M * N;
-  for(int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-      e += (int64_t)gridDim.x * blockDim.x)
-  {
-    int const i = (int)(e / N), j = (int)(e % N);
-    float     v = 0.f;
-    for(int z = 0; z < splits; ++z)
-      v += part[((int64_t)z * M + i) * N + j];
-    v *= alpha;
-    if(accumulate)
-      v += C[i * ldc + j];
-    if(bias)
-      v += bias[j];
-    if(relu)
-      v = v > 0.f ? v : 0.f;
-    C[i * ldc + j] = v;
-  }
-}
-
 // features of cells [cell0, cell0+B): backward differences of orders 0..H-1 of the history
 // (h_1, h_1 - h_2, h_1 - 2 h_2 + h_3, ...), each scaled, then the scaled rhs; targets
 // (optional) = (x_t - extrapolation(h)) * inv_t. The differences are an invertible linear map
@@ -258,34 +140,6 @@ __global__ void __launch_bounds__(256)
   }
   if(threadIdx.x == 0)
     *out = accumulate ? *out + red[0] : red[0];
-}
-
-__global__ void __launch_bounds__(256) relu_backward_kernel(float * dH, float const * H, int64_t n)
-{
-  for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-      i += (int64_t)gridDim.x * blockDim.x)
-    if(H[i] <= 0.f)
-      dH[i] = 0.f;
-}
-
-// db_j = sum_i dY(i,j): one block per column
-__global__ void __launch_bounds__(256) column_sum_kernel(float const * dY, int M, int N, float * db)
-{
-  __shared__ float red[256];
-  int const        j = blockIdx.x;
-  float            s = 0;
-  for(int i = threadIdx.x; i < M; i += 256)
-    s += dY[(int64_t)i * N + j];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for(int w = 128; w > 0; w >>= 1)
-  {
-    if((int)threadIdx.x < w)
-      red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if(threadIdx.x == 0)
-    db[j] = red[0];
 }
 
 __global__ void __launch_bounds__(256)
@@ -642,38 +496,6 @@ inline int grid_for(int64_t n)
 }
 }  // namespace
 
-hipError_t launch_sgemm(int M, int N, int K, float const * A, int64_t a_i, int64_t a_k,
-                        float const * B, int64_t b_k, int64_t b_j, float * C, int64_t ldc,
-                        float alpha, bool accumulate, float const * bias, bool relu,
-                        float * workspace, int64_t workspace_floats, hipStream_t s)
-{
-  int const tiles = ((N + TN - 1) / TN) * ((M + TM - 1) / TM);
-  // split K when the output tiles alone cannot fill the chip (weight gradients: K = batch)
-  int splits = 1;
-  if(workspace != nullptr && tiles < 512 && K >= 8 * TK)
-  {
-    splits = std::min((512 + tiles - 1) / tiles, K / (4 * TK));
-    splits = (int)std::min<int64_t>(splits, workspace_floats / ((int64_t)M * N));
-    splits = std::max(splits, 1);
-  }
-  int const kc = splits > 1 ? ((K + splits - 1) / splits + TK - 1) / TK * TK : K;
-  splits       = (K + kc - 1) / kc;
-  dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, splits);
-  if(splits == 1)
-  {
-    hipLaunchKernelGGL(sgemm_kernel, grid, dim3(256), 0, s, M, N, K, A, a_i, a_k, B, b_k, b_j, C, ldc,
-                       alpha, accumulate ? 1 : 0, bias, relu ? 1 : 0, kc);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(sgemm_kernel, grid, dim3(256), 0, s, M, N, K, A, a_i, a_k, B, b_k, b_j,
-                     workspace, (int64_t)N, 1.f, 0, nullptr, 0, kc);
-  int64_t const total = (int64_t)M * N;
-  int const     g     = (int)std::min<int64_t>((total + 255) / 256, 2048);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(g), dim3(256), 0, s, M, N, splits, workspace, C, ldc,
-                     alpha, accumulate ? 1 : 0, bias, relu ? 1 : 0);
-  return hipGetLastError();
-}
-
 template<typename In>
 hipError_t launch_features(float * X, float * T, History<In> const & hist, In const * rhs,
                            In const * target, int history, int n_cell_dofs, int64_t cell0, int B,
@@ -719,18 +541,6 @@ hipError_t launch_mse_backward(float const * Y, float const * T, float * dY, int
 hipError_t launch_fill_u32(unsigned int * p, unsigned int v, int n, hipStream_t s)
 {
   hipLaunchKernelGGL(fill_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, v, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_relu_backward(float * dH, float const * H, int64_t n, hipStream_t s)
-{
-  hipLaunchKernelGGL(relu_backward_kernel, dim3(grid_for(n)), dim3(256), 0, s, dH, H, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_column_sum(float const * dY, int M, int N, float * db, hipStream_t s)
-{
-  hipLaunchKernelGGL(column_sum_kernel, dim3(N), dim3(256), 0, s, dY, M, N, db);
   return hipGetLastError();
 }
 

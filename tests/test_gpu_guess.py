@@ -71,7 +71,12 @@ def test_extrapolate(torch_cuda, product, order):
 
 
 @pytest.mark.parametrize("degree,history,width,B", [(1, 3, 40, 70), (2, 3, 72, 133), (3, 2, 128, 300),
-                                                    (4, 3, 128, 257), (5, 3, 128, 190)])
+                                                    (4, 3, 128, 257), (5, 3, 128, 190),
+                                                    # the GEMM's tiles and split sums: one sample,
+                                                    # unaligned rows (odd width), the smallest batch
+                                                    # of the largest tile, one past a stage
+                                                    (1, 1, 7, 1), (2, 2, 33, 1025), (1, 4, 128, 16321),
+                                                    (4, 3, 129, 2049)])
 def test_loss_and_grad_vs_oracle(torch_cuda, product, degree, history, width, B):
     torch = torch_cuda
     net = product.GuessNet(degree, history=history, width=width, seed=11)
