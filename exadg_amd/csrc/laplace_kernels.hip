@@ -24,26 +24,47 @@ namespace
 {
 constexpr int cells_per_block(int n) { return (256 / (n * n)) > 0 ? 256 / (n * n) : 1; }
 
-// Base offset and stride of the line along direction d through lane (p,q) of an N^3 block;
-// (p,q) index the two other directions in increasing order.
-template<int N>
+// Base offset and stride of the line along direction d through lane (p,q) of an N^3 block with
+// strides 1, PX, PY; (p,q) index the two other directions in increasing order.
+template<int N, int PX = N, int PY = N * N>
 __device__ __forceinline__ void line_geometry(int d, int p, int q, int & base, int & stride)
 {
   if(d == 0)
   {
-    base   = N * (p + N * q);
+    base   = PX * p + PY * q;
     stride = 1;
   }
   else if(d == 1)
   {
-    base   = p + N * N * q;
-    stride = N;
+    base   = p + PY * q;
+    stride = PX;
   }
   else
   {
-    base   = p + N * q;
-    stride = N * N;
+    base   = p + PX * q;
+    stride = PY;
   }
+}
+
+// face type (kInterior or the boundary type) of side (d, s) of a cell, all six in two bits each, and
+// the face's index; curved meshes keep 6 n^3 metric values per cell, so 32 bits number their faces
+__device__ __forceinline__ int face_types(BoxTopology const & t, int const (&cc)[3])
+{
+  int types = 0;
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
+  {
+    types |= (cc[d] > 0 || t.periodic[d] ? kInterior : t.bc[2 * d]) << (4 * d);
+    types |= (cc[d] < t.nc[d] - 1 || t.periodic[d] ? kInterior : t.bc[2 * d + 1]) << (4 * d + 2);
+  }
+  return types;
+}
+
+__device__ __forceinline__ int face_index(BoxTopology const & t, int const (&cc)[3], int d, int side)
+{
+  int const t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
+  int const fl = cc[d] + side == t.layers[d] ? 0 : cc[d] + side;
+  return (int)t.face_base[d] + fl + t.layers[d] * (cc[t1] + t.nc[t1] * cc[t2]);
 }
 
 // the cell's unit vector in diagonal (probing) mode, else the src line
@@ -70,6 +91,15 @@ __device__ __forceinline__ void source_line(Number const * __restrict__ src, int
 // values, the neighbour traces interpolated from the face nodes, flux with the per-point
 // normal-derivative vectors a = J^{-1} n of both sides, and the face tests added to the
 // Gauss-level residual before the transposed interpolation back to the nodes.
+//
+// What bounds it: the vector-memory address unit (busy 65 - 70% of the cycles), the vector
+// instructions (65% in FP32, 35% in FP64) and the LDS passes (55% / 47%), each waiting on the others
+// between barriers. x-neighbours of the workgroup's row are therefore read from LDS (their strided
+// x-lines cost some 48 address cycles per load), the lanes' rows and columns of Dq come from LDS,
+// the face types and indices are 32-bit and the types taken once, and the LDS strides avoid bank
+// conflicts (GenLayout): FP64 k = 5 on 48^3 cells 651 -> 569 us (3.4 -> 3.9 TB/s of the 2.2 GB it
+// cannot do without), k = 2 on 61 x 47 x 53 167 -> 151 us, FP32 k = 3 on 43 x 37 x 51 89 -> 86 us,
+// the FP32 V-cycle of the k = 5 mesh 7.05 -> 6.37 ms, the same bits.
 
 // FP64 at n = 5, 6: one face direction per round, so that the smaller workspace admits a fourth
 // workgroup per CU
@@ -91,14 +121,32 @@ constexpr bool general_late_gz()
   return !(sizeof(Number) == 8 && N == 8 && mode != ApplyMode::chebyshev);
 }
 
+// LDS strides of a cell: along y (PX) and z (PY) in its tensors, FS from one face array to the
+// next, and S from cell to cell. A group of 16 FP64 (32 FP32) lanes is served in one pass if its
+// addresses differ modulo 16 (32) entries; these are the strides with the fewest passes over the
+// sweeps of the three directions and the face lines that leave the number of workgroups per CU as it
+// is (modeled passes per access 1.4 - 2.3, dense 1.4 - 4.3; at FP64 k = 5 27% and at FP32 34% of
+// the LDS cycles had been conflicts).
 template<int N, typename Number>
-constexpr int general_work_size()
+struct GenLayout
 {
+  static constexpr bool dp = sizeof(Number) == 8;
+  static constexpr int  PX = N == 4 && !dp ? 5 : N;
+  static constexpr int  PY = N == 2 ? 6 : N == 3 ? (dp ? 9 : 13) : N == 4 ? (dp ? 19 : 24) : N == 5 ? 25 :
+                             N == 6 ? (dp ? 39 : 37) : N == 7 ? (dp ? 55 : 49) : N == 8 ? (dp ? 65 : 69) : 81;
+  static constexpr int  FS = N == 4 ? 17 : N == 5 ? (dp ? 25 : 26) : N == 6 ? (dp ? 39 : 36) :
+                             N == 7 ? (dp ? 50 : 49) : N == 8 ? (dp ? 65 : 67) : N == 9 ? 83 : N * N;
+  static constexpr int  S  = N == 2 ? 76 : N == 3 ? (dp ? 171 : 181) : N == 4 ? (dp ? 345 : 364) :
+                             N == 5 ? (dp ? 377 : 569) : N == 6 ? (dp ? 708 : 804) : N == 7 ? (dp ? 1185 : 1137) :
+                             N == 8 ? (dp ? 1559 : 1641) : 2193;
+  static constexpr int  PC = (N - 1) * (PX + PY) + N;
   // cell phase: the x and y gradients (the z one stays in registers); face phases: 8 trace
   // arrays per direction, two directions per round (x and y, then z) or one
-  constexpr int faces = (general_single_rounds<N, Number>() ? 8 : 16) * N * N;
-  return (2 * N * N * N > faces) ? 2 * N * N * N : faces;
-}
+  static constexpr int faces = (general_single_rounds<N, Number>() ? 8 : 16) * FS;
+  static_assert(S >= PC + (2 * PC > faces ? 2 * PC : faces), "cell tensor and workspace");
+  // then the table Dq, whose rows and columns the lanes of the face phases index
+  static constexpr int size = cells_per_block(N) * S + N * N;
+};
 
 // Face terms from the cell's values at the Gauss points. The own traces at the
 // face Gauss points are one dot product per end of the lane's d-line of U (the Gauss values, in
@@ -116,14 +164,14 @@ constexpr int general_work_size()
 // interpolations; the face arrays of direction j live at W + 8 j N^2.
 template<int N, typename Number, ApplyMode mode, int ND>
 __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Number> const & a,
-                                            int64_t cell, int const * cc, bool active, int lt,
-                                            Number const * U, Number * W,
+                                            int64_t cell, int const (&cc)[3], int types, bool active,
+                                            int lt, Number const * U, Number * W, Number const * Dq,
                                             Number const (&nbw)[3][2], Number const (&nbdw)[3][2],
                                             Number (&fr)[3][4])
 {
-  constexpr int  N2 = N * N;
-  using T             = GenTable<N>;
-  Number const * Dq = a.tables + T::DQ;
+  using L           = GenLayout<N, Number>;
+  constexpr int  N2 = N * N, FS = L::FS;
+  using T           = GenTable<N>;
   Number const * d0 = a.tables + T::D0;
   Number const * d1 = a.tables + T::D1;
   Number const * SE = a.tables + T::SE;
@@ -132,36 +180,28 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
   Number const * G0 = a.tables + T::G0;
   Number const * G1 = a.tables + T::G1;
   int const      p = lt % N, q = lt / N;
-  int            type[ND][2];
-#pragma unroll
-  for(int j = 0; j < ND; ++j)
-#pragma unroll
-    for(int s = 0; s < 2; ++s)
-    {
-      int64_t const nb = neighbor_id(a.topo, cc, dirs[j], s);
-      type[j][s]       = nb >= 0 ? kInterior : a.topo.bc[2 * dirs[j] + s];
-    }
+  auto type = [&](int j, int side) { return (types >> (4 * dirs[j] + 2 * side)) & 3; };
   // F1: own traces at the face Gauss points, neighbour traces at the face nodes
   if(active)
 #pragma unroll
     for(int j = 0; j < ND; ++j)
     {
       int const d = dirs[j];
-      Number *  E = W + 8 * j * N2;
+      Number *  E = W + 8 * j * FS;
       int       base, stride;
-      line_geometry<N>(d, p, q, base, stride);
+      line_geometry<N, L::PX, L::PY>(d, p, q, base, stride);
       Number v[N];
       load_line<N>(U + base, stride, v);
-      E[0 * N2 + lt] = dot_line<N>(L0, v);
-      E[1 * N2 + lt] = dot_line<N>(G0, v);
-      E[4 * N2 + lt] = dot_line<N>(L1, v);
-      E[5 * N2 + lt] = dot_line<N>(G1, v);
+      E[0 * FS + lt] = dot_line<N>(L0, v);
+      E[1 * FS + lt] = dot_line<N>(G0, v);
+      E[4 * FS + lt] = dot_line<N>(L1, v);
+      E[5 * FS + lt] = dot_line<N>(G1, v);
       Number nl = 0, dnl = 0, nr = 0, dnr = 0;
       if constexpr(mode != ApplyMode::diagonal)
       {
-        if(type[j][0] == kInterior)
+        if(type(j, 0) == kInterior)
           nl = nbw[d][0], dnl = nbdw[d][0];
-        if(type[j][1] == kInterior)
+        if(type(j, 1) == kInterior)
           nr = nbw[d][1], dnr = nbdw[d][1];
       }
       else
@@ -169,16 +209,17 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
         // probing the cell-local block: neighbours contribute zero, except a cell that is its
         // own periodic neighbour (one cell along d), whose other end then acts as neighbour
         Number u[N];
+        line_geometry<N>(d, p, q, base, stride);
         source_line<N, Number, mode>(a.src, cell, base, stride, a.probe, u);
         if(neighbor_id(a.topo, cc, d, 0) == cell)
           nl = u[N - 1], dnl = dot_line<N>(d1, u);
         if(neighbor_id(a.topo, cc, d, 1) == cell)
           nr = u[0], dnr = dot_line<N>(d0, u);
       }
-      E[2 * N2 + lt] = nl;
-      E[3 * N2 + lt] = dnl;
-      E[6 * N2 + lt] = nr;
-      E[7 * N2 + lt] = dnr;
+      E[2 * FS + lt] = nl;
+      E[3 * FS + lt] = dnl;
+      E[6 * FS + lt] = nr;
+      E[7 * FS + lt] = dnr;
     }
   __syncthreads();
   // F2/F3: the neighbour arrays (slots 2, 3 of each side) to the face Gauss points
@@ -186,7 +227,7 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
     for(int task = lt; task < 4 * ND * N; task += N2)
     {
       int const which = task / N, r = task % N;
-      Number *  arr   = W + (8 * (which >> 2) + 4 * ((which >> 1) & 1) + 2 + (which & 1)) * N2;
+      Number *  arr   = W + (8 * (which >> 2) + 4 * ((which >> 1) & 1) + 2 + (which & 1)) * FS;
       Number    v[N], o[N];
       load_line<N>(arr + N * r, 1, v);
       gen_apply<N, false>(SE, v, o);
@@ -197,7 +238,7 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
     for(int task = lt; task < 4 * ND * N; task += N2)
     {
       int const which = task / N, r = task % N;
-      Number *  arr   = W + (8 * (which >> 2) + 4 * ((which >> 1) & 1) + 2 + (which & 1)) * N2;
+      Number *  arr   = W + (8 * (which >> 2) + 4 * ((which >> 1) & 1) + 2 + (which & 1)) * FS;
       Number    v[N], o[N];
       load_line<N>(arr + r, N, v);
       gen_apply<N, false>(SE, v, o);
@@ -207,6 +248,9 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
   // F4: fluxes at the face quadrature points (side s, point lt), held in registers until
   // every lane has read E
   Number res[ND][2][4];
+  Number D1[N], D2[N];  // the lane's rows of Dq, then its columns
+  load_line<N>(Dq + N * p, 1, D1);
+  load_line<N>(Dq + N * q, 1, D2);
   if(active)
 #pragma unroll
     for(int j = 0; j < ND; ++j)
@@ -216,13 +260,13 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
         int const d = dirs[j];
         int const t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
         int const qq = lt, q1 = qq % N, q2 = qq / N;
-        if(type[j][s] == EXADG_BC_NEUMANN)
+        if(type(j, s) == EXADG_BC_NEUMANN)
         {  // homogeneous Neumann: u+ = u-, du+/dn = -du-/dn -> no contribution
           res[j][s][0] = res[j][s][1] = res[j][s][2] = res[j][s][3] = Number(0);
           continue;
         }
-        int64_t const  f  = face_id(a.topo, cc, d, s);
-        Number const * fd = a.face_data + f * 7 * N2;
+        int const      f  = face_index(a.topo, cc, d, s);
+        Number const * fd = a.face_data + (size_t)f * (7 * N2);
         Number         aK[3], aN[3];
 #pragma unroll
         for(int c = 0; c < 3; ++c)
@@ -232,28 +276,28 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
           aN[c]           = s ? ap : -am;
         }
         Number const   w   = fd[6 * N2 + qq];
-        Number const * Es  = W + 8 * j * N2 + s * 4 * N2;
+        Number const * Es  = W + 8 * j * FS + s * 4 * FS;
         Number         gt1 = 0, gt2 = 0;
 #pragma unroll
         for(int m = 0; m < N; ++m)
         {
-          gt1 += Dq[q1 * N + m] * Es[m + N * q2];
-          gt2 += Dq[q2 * N + m] * Es[q1 + N * m];
+          gt1 += D1[m] * Es[m + N * q2];
+          gt2 += D2[m] * Es[q1 + N * m];
         }
         Number const u      = Es[qq];
-        Number const dudn_K = aK[d] * Es[N2 + qq] + aK[t1] * gt1 + aK[t2] * gt2;
+        Number const dudn_K = aK[d] * Es[FS + qq] + aK[t1] * gt1 + aK[t2] * gt2;
         Number       uN, dudn_N;
-        if(type[j][s] == kInterior)
+        if(type(j, s) == kInterior)
         {
           Number g1 = 0, g2 = 0;
 #pragma unroll
           for(int m = 0; m < N; ++m)
           {
-            g1 += Dq[q1 * N + m] * Es[2 * N2 + m + N * q2];
-            g2 += Dq[q2 * N + m] * Es[2 * N2 + q1 + N * m];
+            g1 += D1[m] * Es[2 * FS + m + N * q2];
+            g2 += D2[m] * Es[2 * FS + q1 + N * m];
           }
-          uN     = Es[2 * N2 + qq];
-          dudn_N = aN[d] * Es[3 * N2 + qq] + aN[t1] * g1 + aN[t2] * g2;
+          uN     = Es[2 * FS + qq];
+          dudn_N = aN[d] * Es[3 * FS + qq] + aN[t1] * g1 + aN[t2] * g2;
         }
         else
         {  // homogeneous Dirichlet: u+ = -u-, du+/dn = du-/dn
@@ -276,9 +320,11 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
       for(int s = 0; s < 2; ++s)
 #pragma unroll
         for(int c = 0; c < 4; ++c)
-          W[(8 * j + 4 * s + c) * N2 + lt] = res[j][s][c];
+          W[(8 * j + 4 * s + c) * FS + lt] = res[j][s][c];
   __syncthreads();
   // F5: tangential gradient tests folded into the value test (Dq^T); this lane's results
+  load_line<N>(Dq + p, N, D1);
+  load_line<N>(Dq + q, N, D2);
   if(active)
 #pragma unroll
     for(int j = 0; j < ND; ++j)
@@ -286,13 +332,13 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
       for(int s = 0; s < 2; ++s)
       {
         int const      qq = lt, q1 = qq % N, q2 = qq / N;
-        Number const * R  = W + (8 * j + 4 * s) * N2;
+        Number const * R  = W + (8 * j + 4 * s) * FS;
         Number         acc = R[qq];
 #pragma unroll
         for(int m = 0; m < N; ++m)
-          acc += Dq[m * N + q1] * R[N2 + m + N * q2] + Dq[m * N + q2] * R[2 * N2 + q1 + N * m];
+          acc += D1[m] * R[FS + m + N * q2] + D2[m] * R[2 * FS + q1 + N * m];
         fr[dirs[j]][2 * s]     = acc;
-        fr[dirs[j]][2 * s + 1] = R[3 * N2 + qq];
+        fr[dirs[j]][2 * s + 1] = R[3 * FS + qq];
       }
   __syncthreads();  // W is reused next
 }
@@ -314,7 +360,8 @@ template<int N, typename Number, ApplyMode mode>
 __global__ void __launch_bounds__(256)
   __attribute__((amdgpu_waves_per_eu(general_min_waves<N, Number>()))) sipg_general_kernel(SipgArgs<Number> a)
 {
-  constexpr int  N2 = N * N, N3 = N * N * N, WS = general_work_size<N, Number>();
+  using L           = GenLayout<N, Number>;
+  constexpr int  N2 = N * N, N3 = N * N * N, PX = L::PX, PY = L::PY;
   constexpr int  CPB = cells_per_block(N);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Number *       smem = reinterpret_cast<Number *>(smem_raw);
@@ -322,18 +369,27 @@ __global__ void __launch_bounds__(256)
   int const      lt   = threadIdx.x - slot * N2;
   int const      pos0 = (int)xcd_logical_block(blockIdx.x, gridDim.x) * CPB;
   bool const     active = slot < CPB && pos0 + slot < (int)a.n_cells;
-  Number *       A      = smem + (active ? slot : 0) * (N3 + WS);
-  Number *       W      = A + N3;
-  Number *       Gx = W, *Gy = W + N3;
+  Number *       A      = smem + (active ? slot : 0) * L::S;
+  Number *       W      = A + L::PC;
+  Number *       Gx = W, *Gy = W + L::PC;
+  Number *       Dq = smem + CPB * L::S;
   Number const * SE  = a.tables + GenTable<N>::SE;
   Number const * DE  = a.tables + GenTable<N>::DE;
   Number const * STE = a.tables + GenTable<N>::STE;
   Number const * DTE = a.tables + GenTable<N>::DTE;
   int const      p = lt % N, q = lt / N;
+  // LDS bases of the lane's x-, y- and z-line
+  int const      bx = PX * p + PY * q, by = p + PY * q, bz = p + PX * q;
   int            cc[3] = {0, 0, 0};
   if(active)
     traversal_coords(a.topo, a.tile_rows, pos0, slot, cc);
-  int64_t const cell = active ? cell_id(a.topo, cc) : 0;
+  int64_t const cell  = active ? cell_id(a.topo, cc) : 0;
+  int const     types = face_types(a.topo, cc);
+  if(threadIdx.x < N2)
+    Dq[threadIdx.x] = a.tables[GenTable<N>::DQ + threadIdx.x];
+  // x-neighbours in the same workgroup are read from its LDS
+  bool const in_block_l = slot > 0 && cc[0] > 0;
+  bool const in_block_r = slot + 1 < CPB && cc[0] + 1 < a.topo.nc[0] && pos0 + slot + 1 < (int)a.n_cells;
 
   // neighbour traces of this lane's line in every direction: value and derivative at the
   // shared face, read up front so that the loads overlap the cell phases
@@ -349,11 +405,15 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
         for(int sd = 0; sd < 2; ++sd)
         {
-          int64_t const nbc = neighbor_id(a.topo, cc, d, sd);
-          if(nbc >= 0)
+          int const n_d = a.topo.nc[d], stride_c = d == 0 ? 1 : d == 1 ? a.topo.nc[0] : a.topo.nc[0] * a.topo.nc[1];
+          bool const wrap = sd ? cc[d] == n_d - 1 : cc[d] == 0;
+          int const  nbc  = (int)cell + (sd ? stride_c : -stride_c) * (wrap ? 1 - n_d : 1);
+          bool const read = ((types >> (4 * d + 2 * sd)) & 3) == kInterior &&
+                            !(d == 0 && (sd ? in_block_r : in_block_l));
+          if(read)
           {
             Number w[N];
-            load_line<N>(a.src + nbc * N3 + base, stride, w);
+            load_line<N>(a.src + (size_t)nbc * N3 + base, stride, w);
             nbw[d][sd]  = sd ? w[0] : w[N - 1];
             nbdw[d][sd] = dot_line<N>(sd ? d0 : d1, w);
           }
@@ -364,32 +424,52 @@ __global__ void __launch_bounds__(256)
   load_traces(1);
   load_traces(2);
 
-  // load the cell values
+  // load the cell values: z-lines of consecutive lanes, consecutive addresses
   if(active)
+#pragma unroll
+    for(int m = 0; m < N; ++m)
+      if constexpr(mode == ApplyMode::diagonal)
+        A[bz + PY * m] = (lt + N2 * m == a.probe) ? Number(1) : Number(0);
+      else
+        A[bz + PY * m] = a.src[cell * N3 + lt + N2 * m];
+  __syncthreads();
+  // nodal -> Gauss values: x, y sweeps in place; the x-neighbours' traces from their nodal lines
+  // before these are overwritten
   {
-    if constexpr(mode == ApplyMode::diagonal)
-      for(int e = lt; e < N3; e += N2)
-        A[e] = (e == a.probe) ? Number(1) : Number(0);
-    else
-      for(int e = lt; e < N3; e += N2)
-        A[e] = a.src[cell * N3 + e];
+    Number v[N], o[N];
+    if(active)
+    {
+      if constexpr(mode != ApplyMode::diagonal)
+      {
+        Number w[N];
+        if(in_block_l)
+        {
+          load_line<N>(A - L::S + bx, 1, w);
+          nbw[0][0]  = w[N - 1];
+          nbdw[0][0] = dot_line<N>(a.tables + GenTable<N>::D1, w);
+        }
+        if(in_block_r)
+        {
+          load_line<N>(A + L::S + bx, 1, w);
+          nbw[0][1]  = w[0];
+          nbdw[0][1] = dot_line<N>(a.tables + GenTable<N>::D0, w);
+        }
+      }
+      load_line<N>(A + bx, 1, v);
+      gen_apply<N, false>(SE, v, o);
+    }
+    if constexpr(mode != ApplyMode::diagonal)
+      __syncthreads();
+    if(active)
+      store_line<N>(A + bx, 1, o);
   }
   __syncthreads();
-  // nodal -> Gauss values: x, y sweeps in place
   if(active)
   {
     Number v[N], o[N];
-    load_line<N>(A + N * (p + N * q), 1, v);
+    load_line<N>(A + by, PX, v);
     gen_apply<N, false>(SE, v, o);
-    store_line<N>(A + N * (p + N * q), 1, o);
-  }
-  __syncthreads();
-  if(active)
-  {
-    Number v[N], o[N];
-    load_line<N>(A + p + N2 * q, N, v);
-    gen_apply<N, false>(SE, v, o);
-    store_line<N>(A + p + N2 * q, N, o);
+    store_line<N>(A + by, PX, o);
   }
   __syncthreads();
   // z sweep, then the z derivative at the Gauss points: this lane's z-line (points lt + m N2),
@@ -401,9 +481,9 @@ __global__ void __launch_bounds__(256)
   if(active)
   {
     Number v[N], o[N];
-    load_line<N>(A + p + N * q, N2, v);
+    load_line<N>(A + bz, PY, v);
     gen_apply<N, false>(SE, v, o);
-    store_line<N>(A + p + N * q, N2, o);
+    store_line<N>(A + bz, PY, o);
     if constexpr(!late_gz)
       gen_apply<N, true>(DE, o, gz_line);
   }
@@ -415,15 +495,15 @@ __global__ void __launch_bounds__(256)
     if constexpr(general_single_rounds<N, Number>())
     {
       int const x[1] = {0}, y[1] = {1}, z[1] = {2};
-      gauss_faces<N, Number, mode, 1>(x, a, cell, cc, active, lt, A, W, nbw, nbdw, fr);
-      gauss_faces<N, Number, mode, 1>(y, a, cell, cc, active, lt, A, W, nbw, nbdw, fr);
-      gauss_faces<N, Number, mode, 1>(z, a, cell, cc, active, lt, A, W, nbw, nbdw, fr);
+      gauss_faces<N, Number, mode, 1>(x, a, cell, cc, types, active, lt, A, W, Dq, nbw, nbdw, fr);
+      gauss_faces<N, Number, mode, 1>(y, a, cell, cc, types, active, lt, A, W, Dq, nbw, nbdw, fr);
+      gauss_faces<N, Number, mode, 1>(z, a, cell, cc, types, active, lt, A, W, Dq, nbw, nbdw, fr);
     }
     else
     {
       int const xy[2] = {0, 1}, z[1] = {2};
-      gauss_faces<N, Number, mode, 2>(xy, a, cell, cc, active, lt, A, W, nbw, nbdw, fr);
-      gauss_faces<N, Number, mode, 1>(z, a, cell, cc, active, lt, A, W, nbw, nbdw, fr);
+      gauss_faces<N, Number, mode, 2>(xy, a, cell, cc, types, active, lt, A, W, Dq, nbw, nbdw, fr);
+      gauss_faces<N, Number, mode, 1>(z, a, cell, cc, types, active, lt, A, W, Dq, nbw, nbdw, fr);
     }
   }
   Number const * L0 = a.tables + GenTable<N>::L0;
@@ -439,15 +519,15 @@ __global__ void __launch_bounds__(256)
   if(active)
   {
     Number v[N], g[N];
-    load_line<N>(A + N * (p + N * q), 1, v);
+    load_line<N>(A + bx, 1, v);
     gen_apply<N, true>(DE, v, g);
-    store_line<N>(Gx + N * (p + N * q), 1, g);
-    load_line<N>(A + p + N2 * q, N, v);
+    store_line<N>(Gx + bx, 1, g);
+    load_line<N>(A + by, PX, v);
     gen_apply<N, true>(DE, v, g);
-    store_line<N>(Gy + p + N2 * q, N, g);
+    store_line<N>(Gy + by, PX, g);
     if constexpr(late_gz)
     {
-      load_line<N>(A + p + N * q, N2, v);
+      load_line<N>(A + bz, PY, v);
       gen_apply<N, true>(DE, v, gz_line);
     }
   }
@@ -459,12 +539,12 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for(int m = 0; m < N; ++m)
     {
-      int const    e  = lt + m * N2;
-      Number const gx = Gx[e], gy = Gy[e], gz = gz_line[m];
+      int const    e  = lt + m * N2, l = bz + m * PY;
+      Number const gx = Gx[l], gy = Gy[l], gz = gz_line[m];
       Number const g00 = G[e], g11 = G[N3 + e], g22 = G[2 * N3 + e];
       Number const g01 = G[3 * N3 + e], g02 = G[4 * N3 + e], g12 = G[5 * N3 + e];
-      Gx[e]            = g00 * gx + g01 * gy + g02 * gz;
-      Gy[e]            = g01 * gx + g11 * gy + g12 * gz;
+      Gx[l]            = g00 * gx + g01 * gy + g02 * gz;
+      Gy[l]            = g01 * gx + g11 * gy + g12 * gz;
       gz_line[m]       = g02 * gx + g12 * gy + g22 * gz;
     }
   }
@@ -473,23 +553,23 @@ __global__ void __launch_bounds__(256)
   if(active)
   {
     Number v[N], o[N];
-    load_line<N>(Gx + N * (p + N * q), 1, v);
+    load_line<N>(Gx + bx, 1, v);
     gen_apply<N, true>(DTE, v, o);
     add_face_tests(o, fr[0]);
-    store_line<N>(A + N * (p + N * q), 1, o);
+    store_line<N>(A + bx, 1, o);
   }
   __syncthreads();
   if(active)
   {
     Number v[N], o[N], w[N];
-    load_line<N>(Gy + p + N2 * q, N, v);
+    load_line<N>(Gy + by, PX, v);
     gen_apply<N, true>(DTE, v, o);
     add_face_tests(o, fr[1]);
-    load_line<N>(A + p + N2 * q, N, w);
+    load_line<N>(A + by, PX, w);
 #pragma unroll
     for(int i = 0; i < N; ++i)
       w[i] += o[i];
-    store_line<N>(A + p + N2 * q, N, w);
+    store_line<N>(A + by, PX, w);
   }
   __syncthreads();
   if(active)
@@ -497,28 +577,28 @@ __global__ void __launch_bounds__(256)
     Number o[N], w[N];
     gen_apply<N, true>(DTE, gz_line, o);
     add_face_tests(o, fr[2]);
-    load_line<N>(A + p + N * q, N2, w);
+    load_line<N>(A + bz, PY, w);
 #pragma unroll
     for(int i = 0; i < N; ++i)
       w[i] += o[i];
     gen_apply<N, false>(STE, w, o);
-    store_line<N>(A + p + N * q, N2, o);
+    store_line<N>(A + bz, PY, o);
   }
   __syncthreads();
   if(active)
   {
     Number v[N], o[N];
-    load_line<N>(A + p + N2 * q, N, v);
+    load_line<N>(A + by, PX, v);
     gen_apply<N, false>(STE, v, o);
-    store_line<N>(A + p + N2 * q, N, o);
+    store_line<N>(A + by, PX, o);
   }
   __syncthreads();
   if(active)
   {
     Number v[N], o[N];
-    load_line<N>(A + N * (p + N * q), 1, v);
+    load_line<N>(A + bx, 1, v);
     gen_apply<N, false>(STE, v, o);
-    store_line<N>(A + N * (p + N * q), 1, o);
+    store_line<N>(A + bx, 1, o);
   }
   __syncthreads();
 
@@ -529,10 +609,11 @@ __global__ void __launch_bounds__(256)
     int const      nc = a.restrict_nc;
     Number const * P  = a.restrict_P;  // P[i nc + c]: fine node i, coarse node c
     Number *       W1 = W;             // nc x N x N
-    Number *       W2 = W + N3;        // nc x nc x N
+    Number *       W2 = W + L::PC;     // nc x nc x N
     if(active)
-      for(int e = lt; e < N3; e += N2)
-        A[e] = a.rhs[cell * N3 + e] - A[e];
+#pragma unroll
+      for(int m = 0; m < N; ++m)
+        A[bz + PY * m] = a.rhs[cell * N3 + lt + N2 * m] - A[bz + PY * m];
     __syncthreads();
     if(active)
     {
@@ -542,7 +623,7 @@ __global__ void __launch_bounds__(256)
         Number s = 0;
 #pragma unroll
         for(int i = 0; i < N; ++i)
-          s += P[i * nc + c] * A[i + N * (j + N * k)];
+          s += P[i * nc + c] * A[i + PX * j + PY * k];
         W1[c + nc * (j + N * k)] = s;
       }
     }
@@ -576,34 +657,33 @@ __global__ void __launch_bounds__(256)
     return;
   }
   if(active)
-  {
-    if constexpr(mode == ApplyMode::diagonal)
+#pragma unroll
+    for(int m = 0; m < N; ++m)
     {
-      if(a.block)
-        for(int e = lt; e < N3; e += N2)
-          a.dst[(cell * N3 + a.probe) * N3 + e] = A[e];
-      else if(lt == 0)
-        a.dst[cell * N3 + a.probe] = A[a.probe];
-    }
-    else if constexpr(mode == ApplyMode::vmult_add)
-      for(int e = lt; e < N3; e += N2)
-        a.dst[cell * N3 + e] += A[e];
-    else if constexpr(mode == ApplyMode::residual)
-      for(int e = lt; e < N3; e += N2)
-        a.dst[cell * N3 + e] = a.rhs[cell * N3 + e] - A[e];
-    else if constexpr(mode == ApplyMode::chebyshev)
-      for(int e = lt; e < N3; e += N2)
+      int const     e  = lt + N2 * m;
+      size_t const  g  = (size_t)cell * N3 + e;
+      Number const  ax = A[bz + PY * m];
+      if constexpr(mode == ApplyMode::diagonal)
       {
-        int64_t const g = cell * N3 + e;
-        Number        v = (Number(1) + a.f1) * a.src[g] + a.f2 * a.dinv[g] * (a.rhs[g] - A[e]);
+        if(a.block)
+          a.dst[((size_t)cell * N3 + a.probe) * N3 + e] = ax;
+        else if(e == a.probe)
+          a.dst[g] = ax;
+      }
+      else if constexpr(mode == ApplyMode::vmult_add)
+        a.dst[g] += ax;
+      else if constexpr(mode == ApplyMode::residual)
+        a.dst[g] = a.rhs[g] - ax;
+      else if constexpr(mode == ApplyMode::chebyshev)
+      {
+        Number v = (Number(1) + a.f1) * a.src[g] + a.f2 * a.dinv[g] * (a.rhs[g] - ax);
         if(a.has_old)
           v -= a.f1 * a.x_old[g];
         a.dst[g] = v;
       }
-    else
-      for(int e = lt; e < N3; e += N2)
-        a.dst[cell * N3 + e] = A[e];
-  }
+      else
+        a.dst[g] = ax;
+    }
 }
 
 template<int N, typename Number, ApplyMode mode>
@@ -611,7 +691,7 @@ hipError_t launch_general_n(SipgArgs<Number> const & a, hipStream_t stream)
 {
   constexpr int CPB    = cells_per_block(N);
   int const     blocks = (int)((a.n_cells + CPB - 1) / CPB);
-  size_t const  lds    = sizeof(Number) * CPB * (N * N * N + general_work_size<N, Number>());
+  size_t const  lds    = sizeof(Number) * GenLayout<N, Number>::size;
   // set once per instantiation; concurrent first calls may both set it, which is harmless
   static std::atomic<bool> attr{false};
   if(lds > 65536 && !attr.load(std::memory_order_acquire))
