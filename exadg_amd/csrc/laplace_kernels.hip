@@ -101,12 +101,13 @@ __device__ __forceinline__ void source_line(Number const * __restrict__ src, int
 // cannot do without), k = 2 on 61 x 47 x 53 167 -> 151 us, FP32 k = 3 on 43 x 37 x 51 89 -> 86 us,
 // the FP32 V-cycle of the k = 5 mesh 7.05 -> 6.37 ms, the same bits.
 
-// FP64 at n = 5, 6: one face direction per round, so that the smaller workspace admits a fourth
-// workgroup per CU
+// FP64 at n = 2, 4, 5, 6: one face direction per round, so that the smaller workspace admits another
+// workgroup per CU (n = 4 on 64^3 cells 502 -> 449 us, n = 2 on 80^3 185 -> 181; n = 3 818 -> 797 on
+// 96^3 but 158 -> 161 on 61 x 47 x 53 and a spill, so it stays)
 template<int N, typename Number>
 constexpr bool general_single_rounds()
 {
-  return sizeof(Number) == 8 && (N == 5 || N == 6);
+  return sizeof(Number) == 8 && N <= 6 && N != 3;
 }
 
 // The z derivative of the Gauss values taken after the face phase, so that it is not held
@@ -136,7 +137,7 @@ struct GenLayout
                              N == 6 ? (dp ? 39 : 37) : N == 7 ? (dp ? 55 : 49) : N == 8 ? (dp ? 65 : 69) : 81;
   static constexpr int  FS = N == 4 ? 17 : N == 5 ? (dp ? 25 : 26) : N == 6 ? (dp ? 39 : 36) :
                              N == 7 ? (dp ? 50 : 49) : N == 8 ? (dp ? 65 : 67) : N == 9 ? 83 : N * N;
-  static constexpr int  S  = N == 2 ? 76 : N == 3 ? (dp ? 171 : 181) : N == 4 ? (dp ? 345 : 364) :
+  static constexpr int  S  = N == 2 ? (dp ? 44 : 76) : N == 3 ? (dp ? 171 : 181) : N == 4 ? (dp ? 219 : 364) :
                              N == 5 ? (dp ? 377 : 569) : N == 6 ? (dp ? 708 : 804) : N == 7 ? (dp ? 1185 : 1137) :
                              N == 8 ? (dp ? 1559 : 1641) : 2193;
   static constexpr int  PC = (N - 1) * (PX + PY) + N;
@@ -344,14 +345,14 @@ __device__ __forceinline__ void gauss_faces(int const (&dirs)[ND], SipgArgs<Numb
 }
 
 // Minimum waves per SIMD asked of the compiler for the general kernel, matched to what the
-// LDS allows: FP64 at n = 3, 5, 6 four (n = 5, 6 with one face direction per round, whose
+// LDS allows: FP64 at n = 2 five, at n = 3..6 four (n = 5, 6 with one face direction per round, whose
 // smaller workspace admits a fourth workgroup per CU: n = 5 8% faster, n = 6 4%); FP32 at n = 3
 // eight (<= 64 VGPRs, 19 KB of LDS per workgroup), at n = 4..6 seven (<= 72 VGPRs), at n = 7 six
 template<int N, typename Number>
 constexpr int general_min_waves()
 {
   if constexpr(sizeof(Number) == 8)
-    return (N == 5 || N == 6) ? 4 : N == 3 ? 4 : 1;
+    return N == 2 ? 5 : N <= 6 ? 4 : 1;
   else
     return N == 3 ? 8 : (N >= 4 && N <= 6) ? 7 : N == 7 ? 6 : 1;
 }
