@@ -34,7 +34,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstddef>
 #include <numeric>
 #include <vector>
 
@@ -96,7 +95,7 @@ __device__ __forceinline__ void store_stream(Number * p, Number v)
   __builtin_nontemporal_store(v, p);
 }
 
-// The 1D tables as uniform (scalar) loads from the kernel arguments. Each phase of the layer loop
+// The 1D tables as uniform (scalar) loads. Each phase of the layer loop
 // takes its pointer anew through fresh(), opaque to the compiler, so that a table is loaded
 // (scalar cache) where it is used: hoisted out of the loop, the tables exceed the scalar
 // registers and are spilled into vector registers.
@@ -246,8 +245,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Number *        smem = reinterpret_cast<Number *>(smem_raw);
   Trace<Number> * halo = reinterpret_cast<Trace<Number> *>(smem + L::cells);
-  static_assert(offsetof(SipgArgs<Number>, tab) == 0, "the tables lead the kernel arguments");
-  Table<Number> const args = (Table<Number>)__builtin_amdgcn_kernarg_segment_ptr();
+  Table<Number> const tables = (Table<Number>)a.tables;
   int const           tid = threadIdx.x, slot = tid / N2, lt = tid - slot * N2;
   int const           nx = a.topo.nc[0], ny = a.topo.nc[1], nz = a.topo.nc[2];
   int const           nxy = nx * ny;
@@ -426,7 +424,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
   {
     if(z0 > 0 || per2)
     {
-      SplitLine<N, Number> const v(args, nxt);
+      SplitLine<N, Number> const v(tables, nxt);
       below = {nxt[N - 1], v.du1};
     }
     if(z0 + 1 < nz || per2)
@@ -439,7 +437,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
   for(int z = z0; z < z1; ++z, g0 += plane)
   {
     // P0
-    Table<Number> tab = fresh<Number>(args);
+    Table<Number> tab = fresh<Number>(tables);
     if(active)
       store_line<N>(smem + bz, L::PY, own);
 #pragma unroll
@@ -454,7 +452,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
     }
     __syncthreads();
     // P1
-    tab = fresh<Number>(args);
+    tab = fresh<Number>(tables);
     Number rx[N];
     // the layers at the ends of the mesh have larger penalties
     bool const end_layer = !per2 && (z < 2 || z >= nz - 2);
@@ -537,7 +535,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
       }
     }
     // P2
-    tab = fresh<Number>(args);
+    tab = fresh<Number>(tables);
     if(opaque(flags[0]) >= 0)
     {
       Number * U = smem + base[0];
@@ -552,7 +550,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
     }
     __syncthreads();
     // P3
-    tab = fresh<Number>(args);
+    tab = fresh<Number>(tables);
     if(opaque(flags[1]) >= 0)
     {
       Number * U = smem + base[1];
@@ -566,7 +564,7 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
     }
     __syncthreads();
     // P4: out = M_z (U + A) + B along z-lines
-    tab = fresh<Number>(args);
+    tab = fresh<Number>(tables);
     Number out[N];
     if(active)
     {
@@ -626,7 +624,7 @@ __global__ void __launch_bounds__(256) sipg_cartesian_kernel(SipgArgs<Number> a)
   constexpr int CPB = 256 / N2;
   using L           = CellLayout<N, Number>;
   using CT          = CartTable<N>;
-  Table<Number> const tab = (Table<Number>)__builtin_amdgcn_kernarg_segment_ptr();
+  Table<Number> const tab = (Table<Number>)a.tables;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Number *      smem   = reinterpret_cast<Number *>(smem_raw);
   int const     slot   = threadIdx.x / N2;
@@ -880,16 +878,6 @@ __global__ void __launch_bounds__(256) sipg_cartesian_kernel(SipgArgs<Number> a)
       }
     }
   }
-}
-
-template<int N, typename Number, ApplyMode mode>
-hipError_t launch_cells_n(SipgArgs<Number> const & a, hipStream_t stream)
-{
-  constexpr int CPB    = 256 / (N * N);
-  int const     blocks = (int)((a.n_cells + CPB - 1) / CPB);
-  size_t const  lds    = sizeof(Number) * CPB * CellLayout<N, Number>::S;
-  hipLaunchKernelGGL((sipg_cartesian_kernel<N, Number, mode>), dim3(blocks), dim3(256), lds, stream, a);
-  return hipGetLastError();
 }
 
 // Whether the layered kernel is the faster one: where its fewer reads count, as src and dst outgrow

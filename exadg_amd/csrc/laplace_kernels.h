@@ -53,13 +53,11 @@ struct CartTable
   static constexpr int line(int d) { return L + d * (cs_size(N) + N); }
 };
 
-// Table layout (Number, SipgArgs::tab): general kernel: [S n*n | Dq n*n | d0 n | d1 n], and in
-// device memory (`tables`) followed by [l(0) n | l(1) n | l'(0) n | l'(1) n] of the Lagrange
-// polynomials on the Gauss points and by the four sweep matrices S, Dq, S^T, Dq^T in even-odd
-// form (GenTable). S is centrosymmetric and Dq skew-centrosymmetric (A_ij = -A_{n-1-i,n-1-j})
-// on the symmetric Gauss points; the skew form stores Ae and Ao as above and, for odd n, the
-// middle row's coefficients of the odd part, A_mj for j < m, padded to m_e entries.
-// Cartesian kernel: CartTable, on the unit interval, plus h per direction.
+// Offsets in the general kernel's table: S n*n, Dq n*n, d0 n, d1 n; l(0), l(1), l'(0), l'(1) of the
+// Lagrange polynomials on the Gauss points, n each; and the four sweep matrices S, Dq, S^T, Dq^T in
+// even-odd form. S is centrosymmetric and Dq skew-centrosymmetric (A_ij = -A_{n-1-i,n-1-j}) on the
+// symmetric Gauss points; the skew form stores Ae and Ao as above and, for odd n, the middle row's
+// coefficients of the odd part, A_mj for j < m, padded to m_e entries.
 template<int N>
 struct GenTable
 {
@@ -70,15 +68,11 @@ struct GenTable
 template<typename Number>
 struct SipgArgs
 {
-  // 1D tables. The Cartesian kernel reads them from this by-value copy, i.e. as uniform scalar
-  // kernel-argument loads (unit-interval mass M, stiffness K, end derivatives d0, d1, scaled
-  // per direction inside the kernel); the general kernel (S, Dq, d0, d1) indexes them at run
-  // time and reads the device copy `tables`.
-  static constexpr int kMaxTable = 4 * cs_size(9) + 5 * 9;
-  Number         tab[kMaxTable];
+  // 1D tables (CartTable, GenTable) in device memory: as a by-value copy in the kernel arguments each
+  // launch wrote them anew and read them past the L2 cache
+  Number const * tables;
   // Cartesian kernel: the scales c_x = h_y h_z, ... of the three Kronecker terms, and c_d/(2 h_d)
   Number         scale[3], half[3];
-  Number const * tables;  // general kernel: the same tables in device memory
   Number const * src;
   Number *       dst;
   Number const * cell_metric;  // general kernel only

@@ -71,9 +71,8 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
   bool const curved = !grid_->affine();
   geo_              = compute_geometry(*grid_, shape_, data.IP_factor, curved);
 
-  // 1D tables travel by value in the kernel arguments (uniform scalar loads); the general
-  // kernel reads the plain layout from device memory
-  std::vector<double> tab, plain;
+  // 1D tables, read by the kernels from device memory
+  std::vector<double> tab;
   auto append = [](std::vector<double> & t, std::vector<double> const & v) {
     t.insert(t.end(), v.begin(), v.end());
   };
@@ -81,6 +80,26 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
   {
     append(tab, shape_.S);
     append(tab, shape_.Dq);
+    append(tab, shape_.d0);
+    append(tab, shape_.d1);
+    // Lagrange polynomials on the Gauss points at the cell ends: values l_q(0), l_q(1), then
+    // derivatives l_q'(0), l_q'(1) (the general kernel's face traces from Gauss values)
+    std::vector<double> v0(n), v1(n), g0(n), g1(n);
+    lagrange_basis(shape_.qp, 0.0, v0.data(), g0.data());
+    lagrange_basis(shape_.qp, 1.0, v1.data(), g1.data());
+    append(tab, v0);
+    append(tab, v1);
+    append(tab, g0);
+    append(tab, g1);
+    // the sweep matrices S, Dq, S^T, Dq^T in even-odd form (GenTable)
+    bool const gp = gen_packed(n);
+    append(tab, even_odd_pack(shape_.S, n, gp, false));
+    append(tab, even_odd_pack(shape_.Dq, n, gp, true));
+    append(tab, even_odd_pack(transposed(shape_.S, n), n, gp, false));
+    append(tab, even_odd_pack(transposed(shape_.Dq, n), n, gp, true));
+    int const size = 2 * n * n + 6 * n + 4 * gen_size(n);
+    if((int)tab.size() != size)
+      EXADG_THROW(EXADG_ERR_INTERNAL, "general-kernel table size");
   }
   else
   {
@@ -117,35 +136,7 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
     if(!map.empty())
       line_map_.upload(map);
   }
-  append(plain, curved ? shape_.S : shape_.mass);
-  append(plain, curved ? shape_.Dq : shape_.stiff);
-  append(plain, shape_.d0);
-  append(plain, shape_.d1);
-  if(curved)
-  {
-    // Lagrange polynomials on the Gauss points at the cell ends: values l_q(0), l_q(1), then
-    // derivatives l_q'(0), l_q'(1) (the general kernel's face traces from Gauss values)
-    std::vector<double> v0(n), v1(n), g0(n), g1(n);
-    lagrange_basis(shape_.qp, 0.0, v0.data(), g0.data());
-    lagrange_basis(shape_.qp, 1.0, v1.data(), g1.data());
-    append(plain, v0);
-    append(plain, v1);
-    append(plain, g0);
-    append(plain, g1);
-    // the sweep matrices S, Dq, S^T, Dq^T in even-odd form (GenTable)
-    bool const gp = gen_packed(n);
-    append(plain, even_odd_pack(shape_.S, n, gp, false));
-    append(plain, even_odd_pack(shape_.Dq, n, gp, true));
-    append(plain, even_odd_pack(transposed(shape_.S, n), n, gp, false));
-    append(plain, even_odd_pack(transposed(shape_.Dq, n), n, gp, true));
-    int const size = 2 * n * n + 6 * n + 4 * gen_size(n);
-    if((int)plain.size() != size)
-      EXADG_THROW(EXADG_ERR_INTERNAL, "general-kernel table size");
-  }
-  if((int)tab.size() > SipgArgs<Number>::kMaxTable)
-    EXADG_THROW(EXADG_ERR_INTERNAL, "1D tables exceed the kernel-argument table");
-  tab_.assign(tab.begin(), tab.end());
-  tables_.upload(std::vector<Number>(plain.begin(), plain.end()));
+  tables_.upload(std::vector<Number>(tab.begin(), tab.end()));
   if(!curved)
   {
     // unit-interval 1D diagonals and end derivatives of the closed-form diagonal
@@ -242,7 +233,6 @@ template<typename Number>
 SipgArgs<Number> LaplaceOperator<Number>::make_args(Number * dst, Number const * src, int probe) const
 {
   SipgArgs<Number> a;
-  std::copy(tab_.begin(), tab_.end(), a.tab);
   std::copy(scale_, scale_ + 3, a.scale);
   std::copy(half_, half_ + 3, a.half);
   a.tables      = tables_.data();

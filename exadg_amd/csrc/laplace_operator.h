@@ -173,7 +173,6 @@ private:
   ShapeInfo1D                           shape_;
   GeometryData                          geo_;  // host copy (tau, and metric for curved)
   int                                   n3_;
-  std::vector<Number>                   tab_;  // 1D tables (kernel-argument copy)
   Number                                scale_[3] = {1, 1, 1}, half_[3] = {1, 1, 1};
   DeviceBuffer<Number>                  tables_, cell_metric_, face_data_, tau_face_;
   DeviceBuffer<int>                     line_map_;            // cartesian_line_map
