@@ -1,6 +1,7 @@
 #include "multigrid.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <string>
@@ -359,14 +360,62 @@ Q1Operator<Number>::Q1Operator(StructuredGrid const & grid) : topo_(grid.topolog
       }
     }
   });
-  stencil_.upload(std::vector<Number>(W.begin(), W.end()));
+  // the rows by node class where they are the same bits for every node of a class, which shared
+  // element matrices give, and the planes are long
+  std::vector<Number> classes;
+  if(grid.affine() && nn * (int64_t)(27 * sizeof(Number)) >= kQ1ClassBytes)
+    classes = stencil_classes(W);
+  if(!classes.empty())
+    classes_.upload(classes);
+  else
+    stencil_.upload(std::vector<Number>(W.begin(), W.end()));
   diag_.upload(std::vector<Number>(D.begin(), D.end()));
+}
+
+template<typename Number>
+std::vector<Number> Q1Operator<Number>::stencil_classes(std::vector<double> const & W) const
+{
+  // the class of coordinate c in direction d, and a coordinate of class k or -1
+  auto kind = [&](int d, int c) {
+    int const m = q_.nn[d];
+    return q_.periodic[d] ? 2 : m < 5 || c < 2 ? c : c >= m - 2 ? c + 5 - m : 2;
+  };
+  auto member = [&](int d, int k) {
+    int const m = q_.nn[d];
+    if(q_.periodic[d])
+      return k == 2 ? 0 : -1;
+    return m < 5 ? (k < m ? k : -1) : k <= 2 ? k : k + m - 5;
+  };
+  int64_t const       nn = n_nodes_;
+  std::vector<double> t((size_t)kQ1Classes * kQ1ClassStride, 0.0);
+  for(int c = 0; c < kQ1Classes; ++c)
+  {
+    int const x = member(0, c % 5), y = member(1, c / 5 % 5), z = member(2, c / 25);
+    if(x < 0 || y < 0 || z < 0)
+      continue;
+    int64_t const node = x + (int64_t)q_.nn[0] * (y + (int64_t)q_.nn[1] * z);
+    for(int j = 0; j < 27; ++j)
+      t[c * kQ1ClassStride + j] = W[(size_t)j * nn + node];
+  }
+  std::atomic<bool> same(true);
+  parallel_range(nn, [&](int64_t nb, int64_t ne) {
+    for(int64_t node = nb; node < ne; ++node)
+    {
+      int const c = kind(0, (int)(node % q_.nn[0])) +
+                    5 * (kind(1, (int)((node / q_.nn[0]) % q_.nn[1])) +
+                         5 * kind(2, (int)(node / ((int64_t)q_.nn[0] * q_.nn[1]))));
+      for(int j = 0; j < 27; ++j)
+        if(W[(size_t)j * nn + node] != t[c * kQ1ClassStride + j])
+          same = false;
+    }
+  });
+  return same ? std::vector<Number>(t.begin(), t.end()) : std::vector<Number>();
 }
 
 template<typename Number>
 void Q1Operator<Number>::vmult(Number * dst, Number const * src, hipStream_t s) const
 {
-  hipError_t e = launch_q1_stencil<Number>(dst, src, stencil_.data(), q_, s);
+  hipError_t e = launch_q1_stencil<Number>(dst, src, weights(), q_, s);
   if(e != hipSuccess)
     EXADG_THROW(EXADG_ERR_HIP, hipGetErrorString(e));
 }
@@ -377,7 +426,7 @@ bool Q1Operator<Number>::chebyshev_step(Number * x_new, Number const * x, Number
                                         bool has_old, hipStream_t s) const
 {
   hipError_t e =
-    launch_q1_chebyshev<Number>(x_new, x, x_old, b, dinv, stencil_.data(), q_, f1, f2, has_old, s);
+    launch_q1_chebyshev<Number>(x_new, x, x_old, b, dinv, weights(), q_, f1, f2, has_old, s);
   if(e != hipSuccess)
     EXADG_THROW(EXADG_ERR_HIP, hipGetErrorString(e));
   return true;

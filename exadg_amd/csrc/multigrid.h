@@ -218,12 +218,16 @@ public:
   std::vector<double> const & element_matrices() const { return mats_host_; }
 
 private:
+  // the stencil's rows by node class; empty if the nodes of a class differ
+  std::vector<Number> stencil_classes(std::vector<double> const & W) const;
+  Q1Weights<Number>   weights() const { return {stencil_.data(), classes_.data()}; }
+
   BoxTopology          topo_;
   Q1Topology           q_;
   CGTopology           cg_;
   int64_t              n_nodes_;
   std::vector<double>  mats_host_;  // 8x8 element matrices (one shared one if affine)
-  DeviceBuffer<Number> stencil_;    // assembled 27-point stencil, 27 planes of n_nodes
+  DeviceBuffer<Number> stencil_, classes_;  // 27-point stencil per node and per class (Q1Weights)
   DeviceBuffer<Number> diag_;       // sum over cells of K_vv (1 on constrained rows)
 };
 

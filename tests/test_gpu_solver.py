@@ -115,6 +115,38 @@ def test_coarse_pcg_matches_oracle(nc, per, bc, nodes, torch_cuda, product):
     assert e.value.code == product.EXADG_ERR_NOT_FINITE
 
 
+# Q1 levels of affine boxes just long enough for node classes in FP32, with 1, 2, 4, 5 and more
+# nodes per direction and waves of one class and of several; a Dirichlet side of a short direction
+# keeps the number of Chebyshev steps small
+Q1_CLASSES = [
+    ((1, 4, 18519), (0, 0, 0), (D, N, N, D, N, N)),
+    ((3, 5, 7800), (0, 0, 0), (D,) * 6),
+    ((4, 3, 11600), (1, 0, 0), (N, N, D, N, D, D)),
+    ((300, 25, 24), (1, 0, 0), (N, N, D, N, N, D)),
+    ((1, 46300, 3), (1, 0, 0), (N, N, N, N, D, N)),
+]
+
+
+@pytest.mark.parametrize("nc,per,bc", Q1_CLASSES, ids=[str(c[0]) for c in Q1_CLASSES])
+def test_q1_stencil_classes_match_oracle(nc, per, bc, torch_cuda, product):
+    """The V-cycle over DG 1 and the Q1 level smoothed by Chebyshev steps, with the bars above."""
+    torch = torch_cuda
+    up = tuple(n / 10 for n in nc)
+    mg_o = oracle.Multigrid(oracle.make_mesh(nc, 0.0, up, periodic=per, boundary_type=bc), [1],
+                            coarse_solver=1)
+    op = product.LaplaceOperator(product.mesh_desc(nc, 0.0, up, periodic=per), product.bc_desc(bc), 1)
+    r = oracle.random_vector(op.n)
+    z_ref = mg_o.vmult(r)
+    z = torch.empty(op.n, dtype=torch.float64, device="cuda")
+    for precision, bar in ((product.FP64, 1e-9), (product.FP32, 1e-4)):
+        prec = product.Preconditioner(op, product.PRECOND_MULTIGRID, product.mg_desc(
+            1, degrees=[1], precision=precision, coarse_solver=1))
+        prec.vmult(z, torch.from_numpy(r).cuda())
+        err = _rel(z.cpu().numpy(), z_ref)
+        print(f"{nc}: V-cycle rel.err {err:.2e}", flush=True)
+        assert err <= bar
+
+
 @pytest.mark.parametrize("case", MG_CASES[:2], ids=[c[0] for c in MG_CASES[:2]])
 def test_vcycle_fp32_close_to_oracle(case, torch_cuda, product):
     torch = torch_cuda
