@@ -357,21 +357,17 @@ def main():
         "config": {"workload": f"SIPG vmult, affine Cartesian [0,1]^3, {args.cells}^3 cells, "
                                f"degree {args.degree}, FP64, homogeneous Dirichlet",
                    "n_dofs": n, "n_cells": op.n_cells, "degree": args.degree,
-                   "kernel": "sipg_cartesian_kernel",
+                   "kernel": "sipg_cartesian_layers_kernel",
                    "kernel_ms_mean": round(statistics.mean(kernel_ms), 5),
                    "kernel_ms_median": round(statistics.median(kernel_ms), 5),
                    "kernel_ms_min": round(min(kernel_ms), 5)},
-        # the roofline of a streaming operator is HBM; what holds this kernel below it is the
-        # latency of each workgroup's chain (loads, LDS staging, five dependent LDS phases,
-        # store), overlapped only partly across the resident workgroups: the VALU is busy ~40%
-        # of the time, half of each wave's life is spent in waits, and probes removing VALU
-        # work, barriers or LDS traffic each gain only a few percent
+        # the roofline of a streaming operator is HBM; what holds this kernel below it are LDS
+        # passes, vector-memory addresses and vector instructions, each busy for much of the time
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "limiter": "latency of the per-workgroup load -> LDS phases -> store chain, "
-                                "not HBM bytes (traffic ~1.2x algorithmic) nor VALU/LDS "
-                                "throughput"},
+                     "limiter": "LDS passes, vector-memory addresses and VALU work together, "
+                                "not HBM bytes (traffic ~1.26x algorithmic)"},
         "stream": stream_bw,
     }
     if not args.no_solve:
