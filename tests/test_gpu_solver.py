@@ -147,6 +147,27 @@ def test_q1_stencil_classes_match_oracle(nc, per, bc, torch_cuda, product):
         assert err <= bar
 
 
+@pytest.mark.parametrize("nc", [(9, 8, 11), (10, 9, 7), (12, 11, 13)], ids=str)
+def test_vcycle_fp32_has_no_scale(nc, torch_cuda, product):
+    """A Chebyshev step leaves x = x_old alone up to D^-1 (b - A x): with coefficients 1 + f1 and f1
+    that differ by 1 only up to rounding, each of the 9 steps of the 4 levels scales the iterate by up
+    to 6e-8, always the same way. What is left is the rounding of the vectors, 36 steps of 6e-8 at
+    random (4e-7 in the norm), of which the scale, one component, sees a small part."""
+    torch = torch_cuda
+    op = product.LaplaceOperator(product.mesh_desc(nc), product.bc_desc((D, N) + (D,) * 4), 5)
+    b = torch.from_numpy(oracle.random_vector(op.n)).cuda()
+    z = []
+    for precision in (product.FP32, product.FP64):
+        prec = product.Preconditioner(op, product.PRECOND_MULTIGRID, product.mg_desc(
+            5, degrees=[5, 3, 2, 1], precision=precision, coarse_solver=product.COARSE_CHEBYSHEV))
+        z.append(torch.empty_like(b))
+        prec.vmult(z[-1], b)
+    d = z[0] - z[1]
+    scale = float(d @ z[1] / (z[1] @ z[1]))
+    print(f"{nc}: scale {scale:.2e}, rel. difference {float(d.norm() / z[1].norm()):.2e}", flush=True)
+    assert abs(scale) <= 3e-7
+
+
 @pytest.mark.parametrize("case", MG_CASES[:2], ids=[c[0] for c in MG_CASES[:2]])
 def test_vcycle_fp32_close_to_oracle(case, torch_cuda, product):
     torch = torch_cuda
