@@ -56,6 +56,39 @@ std::vector<double> transposed(std::vector<double> const & A, int n)
       t[j * n + i] = A[i * n + j];
   return t;
 }
+
+// A row t of n entries that vanishes on constants (of the even part of a line: twice its values, and
+// once the middle one, the last if n is odd for the line), rounded to Number such that it still does:
+// the smallest entry, whose last place is the finest, takes up what rounding left. A row that
+// keeps 1e-8 of a constant looks like a reaction term, which counts where u is smooth and A u small.
+template<typename Number>
+void round_zero_sum(double * t, int n, bool even_part, bool middle)
+{
+  auto weight = [&](int j) { return even_part && !(middle && j == n - 1) ? 2 : 1; };
+  int  k      = 0;
+  for(int j = 0; j < n; ++j)
+  {
+    t[j] = (Number)t[j];
+    if(std::abs(t[j]) < std::abs(t[k]))
+      k = j;
+  }
+  long double sum = 0;
+  for(int j = 0; j < n; ++j)
+    if(j != k)
+      sum += weight(j) * (long double)t[j];
+  t[k] = (Number)(-sum / weight(k));
+}
+
+// the same for the even part of a packed matrix, row by row (even_odd_pack)
+template<typename Number>
+void round_zero_sums(std::vector<double> & packed, int n)
+{
+  int const m = n / 2, me = m + n % 2;
+  for(int i = 0; i < m; ++i)
+    round_zero_sum<Number>(packed.data() + i * me, me, true, n % 2);
+  if(n % 2)
+    round_zero_sum<Number>(packed.data() + m * me + m * m, me, true, true);
+}
 }  // namespace
 
 template<typename Number>
@@ -105,7 +138,7 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
   {
     // the end derivative d0 in even-odd form (CartTable); d1 mirrors it
     int const           m = n / 2;
-    std::vector<double> de, scaled;
+    std::vector<double> de, scaled, d0 = shape_.d0;
     for(int j = 0; j < n; ++j)
       if(std::abs(shape_.d1[j] + shape_.d0[n - 1 - j]) > 1e-12 * std::abs(shape_.d0[0]))
         EXADG_THROW(EXADG_ERR_INTERNAL, "the 1D end derivatives do not mirror each other");
@@ -116,8 +149,11 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
     for(int j = 0; j < m; ++j)
       de.push_back(0.5 * (shape_.d0[j] - shape_.d0[n - 1 - j]));
     append(tab, even_odd_pack(shape_.mass, n, true, false));
-    append(tab, shape_.d0);
-    append(tab, de);
+    round_zero_sum<Number>(d0.data(), n, false, false);
+    append(tab, d0);
+    scaled = de;
+    round_zero_sum<Number>(scaled.data(), m + n % 2, true, n % 2);
+    append(tab, scaled);
     for(int d = 0; d < 3; ++d)
     {
       double const c = grid_->h((d + 1) % 3) * grid_->h((d + 2) % 3), s = c / grid_->h(d);
@@ -126,10 +162,12 @@ LaplaceOperator<Number>::LaplaceOperator(std::shared_ptr<StructuredGrid const> g
       scaled         = even_odd_pack(shape_.stiff, n, true, false);
       for(double & v : scaled)
         v *= s;
+      round_zero_sums<Number>(scaled, n);
       append(tab, scaled);
       scaled = de;
       for(double & v : scaled)
         v *= 0.5 * s;
+      round_zero_sum<Number>(scaled.data(), m + n % 2, true, n % 2);
       append(tab, scaled);
     }
     std::vector<int> const map = cartesian_line_map<Number>(data.degree);

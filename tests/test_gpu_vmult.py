@@ -70,6 +70,33 @@ def test_vmult_fp64_matches_oracle(case, torch_cuda, product):
     assert _rel(ys.cpu().numpy(), 2 * y_ref) <= 1e-12
 
 
+@pytest.mark.parametrize("k", range(2, 9))
+def test_fp32_rows_vanish_on_constants(k, torch_cuda, product):
+    """The FP32 affine operator on smooth fields, relative to FP64 by u.(A32 - A64)u / u.A64 u. Rounded
+    1D stiffness rows whose entries (up to K) do not add up to zero keep up to 2^-25 K of a constant each; the
+    n rows of a cell add up to n 2^-25 K / h^2 per direction against an eigenvalue of (2 pi)^2 per
+    direction: 9e-6 at k = 4 and 6e-5 at k = 8 for h = 1/14 (2e-6 to 3e-5 were seen). Rows that
+    vanish on constants leave the rounding of the sums, whose sign changes with u: below 2e-6."""
+    torch = torch_cuda
+    err = []
+    for nc in ((14, 13, 15), (16, 16, 16), (11, 17, 12), (13, 18, 10)):
+        mesh, bc = product.mesh_desc(nc), product.bc_desc((N,) * 6)
+        a32 = product.LaplaceOperator(mesh, bc, k, product.FP32)
+        a64 = product.LaplaceOperator(mesh, bc, k, product.FP64)
+        nodes = torch.from_numpy(np.ascontiguousarray(oracle.tables(k)["gl"])).cuda()
+        x = [(torch.arange(n, dtype=torch.float64, device="cuda")[:, None] + nodes) / n for n in nc]
+        c = [torch.cos(2 * np.pi * v + 0.1) for v in x]
+        u = (c[2][:, None, None, :, None, None] * c[1][None, :, None, None, :, None]
+             * c[0][None, None, :, None, None, :]).float().reshape(-1)
+        y, r = torch.empty_like(u), torch.empty(a64.n, dtype=torch.float64, device="cuda")
+        a32.vmult(y, u)
+        u = u.double()
+        a64.vmult(r, u)
+        err.append(float(u @ (y.double() - r) / (u @ r)))
+    print(f"k{k}: " + " ".join(f"{e:.1e}" for e in err), flush=True)
+    assert np.sqrt(np.mean(np.square(err))) <= 2e-6
+
+
 # affine meshes just above the sizes where the layered kernel takes over (15 and 60 MB a vector in
 # FP32, 90 MB in FP64): rows that end inside a tile, odd last rows of tiles, segments of unequal
 # length, a box shorter than a tile, one layer, and every periodic direction
