@@ -26,8 +26,9 @@ struct FeatureScales
 
 // C(i,j) = alpha sum_k A(i,k) B(k,j) (+ C if accumulate) (+ bias_j) (ReLU) (0 where mask(i,j) <= 0,
 // laid out as C), A(i,k) = A[i a_i + k a_k], B(k,j) = B[k b_k + j b_j], one of the two strides of
-// each being 1; row_sum (if not null) receives sum_k A(i,k). With a workspace of >= s M (N + 1)
-// floats the K range may be split over s blocks when M x N alone has too few tiles.
+// each being 1 (not a_i with b_k alone); row_sum (if not null) receives sum_k A(i,k). With a
+// workspace (gradients: sums over the batch) of >= s M (N + 1) floats the K range may be split over s
+// blocks when M x N alone has too few tiles, and the sums are taken in short chains.
 struct SgemmArgs
 {
   int           M, N, K;

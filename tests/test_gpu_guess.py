@@ -99,6 +99,36 @@ def test_loss_and_grad_vs_oracle(torch_cuda, product, degree, history, width, B)
         assert np.max(np.abs(blk)) > 0
 
 
+@pytest.mark.parametrize("degree,B", [(2, 2048), (2, 4096), (3, 3001), (3, 4096), (4, 4096)])
+def test_gradient_sums_are_short_chains(torch_cuda, product, degree, B):
+    """Rounding of the sums over the batch in the last layer's gradient. The biases are added in FP64: a
+    rounding of 2^-24 / sqrt(3) = 3.4e-8 in the parts' sums, in the result and in dY, 6e-8 together.
+    The weights are added in chains of 64 products: 3.4e-8 sqrt(64 / 2) = 1.9e-7 of a chain, averaged
+    over B / 64 chains (3.4e-8 at 2048), then as much for each of the sums of chains, the result, dY and
+    H2: 8e-8 (asked at degree 2, where the forward pass has short sums too). With one chain per
+    part the biases have 0.7 - 1.0e-7 and the weights 9.4e-8 at 4096 and 9.9e-8 at 2048."""
+    torch = torch_cuda
+    net = product.GuessNet(degree, history=3, width=128, seed=11)
+    n3 = (degree + 1) ** 3
+    err = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        p = np.concatenate([rng.uniform(-b, b, n) for n, b in (
+            (128 * 4 * n3, (6 / (4 * n3)) ** 0.5), (128, 0.1), (128 * 128, (6 / 128) ** 0.5), (128, 0.1),
+            (n3 * 128, 0.1 * (6 / 128) ** 0.5), (n3, 0.1))]).astype(np.float32)
+        net.set_params(torch.from_numpy(p))
+        X = rng.uniform(-1, 1, (B, net.n_features)).astype(np.float32)
+        T = rng.uniform(-1, 1, (B, n3)).astype(np.float32)
+        _, g = net.loss_and_grad(torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda())
+        _, go = og.loss_and_grad(p.astype(np.float64), X.astype(np.float64), T.astype(np.float64), 128, n3)
+        got, ref = (og.unpack(v, net.n_features, 128, n3) for v in (g.cpu().numpy().astype(np.float64), go))
+        err.append([np.linalg.norm(got[i] - ref[i]) / np.linalg.norm(ref[i]) for i in (4, 5)])
+    W3, b3 = np.sqrt(np.mean(np.square(err), axis=0))
+    print(f"k{degree} B{B}: W3 {W3:.2e} b3 {b3:.2e}", flush=True)
+    assert b3 <= 6e-8
+    assert degree > 2 or W3 <= 8e-8
+
+
 def _sequence(torch, product, n_cells, degree, n_steps, k_max=3, dt=0.01, seed=5):
     from exadg_amd import pressure_sequence as ps
     op, prec = ps.setup_box(product, n_cells, degree, product.FP32)
