@@ -116,15 +116,27 @@ struct alignas(2 * sizeof(Number)) Trace
   Number w, dw;
 };
 
+// sum_i a_i v_{n-1-i}
+template<int N, typename Number>
+__device__ __forceinline__ Number dot_reversed(Table<Number> const a, Number const (&v)[N])
+{
+  Number s = 0;
+#pragma unroll
+  for(int i = 0; i < N; ++i)
+    s += a[i] * v[N - 1 - i];
+  return s;
+}
+
 // A line split into its even part e (v_j + v_{n-1-j}, the middle value last for odd n) and odd part
 // o (v_j - v_{n-1-j}), with its end derivatives du(0), du(1): on symmetric nodes they mirror each
 // other (d1_i = -d0_{n-1-i}), so that du(0) = de + do and du(1) = do - de with the even-odd form
-// of d0
+// of d0. FP64 at n = 7 takes them by plain products instead, which measured 2% faster (see CellLayout).
 template<int N, typename Number>
 struct SplitLine
 {
-  static constexpr int m = N / 2, me = m + N % 2;
-  Number               e[me], o[m], du0, du1;
+  static constexpr int  m = N / 2, me = m + N % 2;
+  static constexpr bool plain = sizeof(Number) == 8 && N == 7;
+  Number                e[me], o[m], du0, du1;
   __device__ __forceinline__ SplitLine(Table<Number> const tab, Number const (&v)[N])
   {
     Table<Number> const DE = tab + CartTable<N>::DE, DO = tab + CartTable<N>::DO;
@@ -134,16 +146,20 @@ struct SplitLine
     {
       e[j] = v[j] + v[N - 1 - j];
       o[j] = v[j] - v[N - 1 - j];
-      se += DE[j] * e[j];
-      so += DO[j] * o[j];
+      if constexpr(!plain)
+      {
+        se += DE[j] * e[j];
+        so += DO[j] * o[j];
+      }
     }
     if constexpr(N % 2 == 1)
     {
       e[m] = v[m];
-      se += DE[m] * e[m];
+      if constexpr(!plain)
+        se += DE[m] * e[m];
     }
-    du0 = se + so;
-    du1 = so - se;
+    du0 = plain ? dot_line<N>(tab + CartTable<N>::D0, v) : se + so;
+    du1 = plain ? -dot_reversed<N, Number>(tab + CartTable<N>::D0, v) : so - se;
   }
 };
 
@@ -186,17 +202,6 @@ __device__ __forceinline__ void line_laplacian(Table<Number> const L, Number hal
   out[0] += tau_l * jl;
   out[N - 1] -= half * (u.du1 + r.dw);
   out[N - 1] += tau_r * jr;
-}
-
-// sum_i a_i v_{n-1-i}
-template<int N, typename Number>
-__device__ __forceinline__ Number dot_reversed(Table<Number> const a, Number const (&v)[N])
-{
-  Number s = 0;
-#pragma unroll
-  for(int i = 0; i < N; ++i)
-    s += a[i] * v[N - 1 - i];
-  return s;
 }
 
 // the exterior trace of a boundary face from the line's own trace (weak_boundary_conditions.h)
@@ -597,20 +602,23 @@ __global__ void __launch_bounds__((CartTile<N, Number>::threads))
 // group of 16 FP64 (32 FP32) lanes is served in one pass if its addresses differ modulo 16 (32)
 // entries; these are the strides with the fewest passes over the three directions that leave the
 // number of workgroups per CU as it is (modeled passes per access 1.26 - 1.61 instead of 1.5 - 4.1
-// dense).
+// dense). FP64 at n = 7 keeps wider strides with more modeled passes: with PY = 49, S = 1041, the
+// x-lines swapped and even-odd end derivatives vmult and vmult_add took 2 - 6% longer on 16^3 to
+// 32 x 31 x 30 cells (24 x 23 x 22: 32.4 / 31.4 us, vmult_add 34.9 / 33.8), most of it from the
+// strides; both leave three workgroups per CU.
 template<int N, typename Number>
 struct CellLayout
 {
   static constexpr bool dp = sizeof(Number) == 8;
   static constexpr int  PX = N == 2 ? 3 : N == 4 ? 5 : N;
-  static constexpr int  PY = N == 2 ? 6 : N == 4 ? 20 : N == 6 ? (dp ? 41 : 37) : N == 7 ? (dp ? 49 : 52) :
+  static constexpr int  PY = N == 2 ? 6 : N == 4 ? 20 : N == 6 ? (dp ? 41 : 37) : N == 7 ? 52 :
                              N == 8 ? (dp ? 65 : 67) : N * N;
   static constexpr int  PC = (N - 1) * (PX + PY) + N;
   static constexpr int  S  = N == 2 ? 36 : N == 3 ? 91 : N == 4 ? (dp ? 237 : 240) : N == 5 ? 381 :
-                             N == 6 ? (dp ? 724 : 676) : N == 7 ? (dp ? 1041 : 1105) :
+                             N == 6 ? (dp ? 724 : 676) : N == 7 ? (dp ? 1107 : 1105) :
                              N == 8 ? (dp ? 1557 : 1599) : dp ? 2193 : 2201;
   static_assert(S >= 3 * PC, "three buffers per cell");
-  static constexpr bool swap_x = dp ? N >= 6 : N == 7 || N == 8;
+  static constexpr bool swap_x = dp ? N == 6 || N >= 8 : N == 7 || N == 8;
   static constexpr bool swap_y = !dp && (N == 6 || N == 8);
 };
 
