@@ -153,6 +153,7 @@ def lib():
             "exadg_laplace_destroy": [vp],
             "exadg_laplace_n_dofs": [vp, i64p],
             "exadg_laplace_info": [vp, i64p, ip, ip, ip],
+            "exadg_laplace_kernel": [vp, ctypes.POINTER(ctypes.c_char_p)],
             "exadg_laplace_vmult": [vp, vp, vp, vp],
             "exadg_laplace_vmult_add": [vp, vp, vp, vp],
             "exadg_laplace_calculate_inverse_diagonal": [vp, vp, vp],
@@ -269,6 +270,13 @@ class LaplaceOperator:
     @property
     def handle(self):
         return self._h
+
+    @property
+    def kernel(self):
+        """Name of the kernel that vmult and vmult_add launch."""
+        name = ctypes.c_char_p()
+        check(lib().exadg_laplace_kernel(self._h, ctypes.byref(name)))
+        return name.value.decode()
 
     def close(self):
         if getattr(self, "_h", None) and self._h.value:

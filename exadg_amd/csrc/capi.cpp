@@ -275,6 +275,14 @@ int exadg_laplace_info(const exadg_laplace * op, int64_t * n_cells, int * degree
   });
 }
 
+int exadg_laplace_kernel(const exadg_laplace * op, const char ** name)
+{
+  return guarded([&] {
+    require(op && name, "null argument");
+    *name = op->op->vmult_kernel();
+  });
+}
+
 int exadg_laplace_vmult(exadg_laplace * op, void * dst, const void * src, void * stream)
 {
   return guarded([&] {

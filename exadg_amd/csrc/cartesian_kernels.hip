@@ -888,36 +888,65 @@ __global__ void __launch_bounds__(256) sipg_cartesian_kernel(SipgArgs<Number> a)
   }
 }
 
+// How the layered kernel covers a box: tiles of BX columns of the rows of BY cells, laid end to end,
+// and segments of layers
+struct LayerTiling
+{
+  int row_length, tiles, segments, layers_per_segment;
+};
+
+template<int N, typename Number>
+LayerTiling layer_tiling(BoxTopology const & t)
+{
+  using Tile   = CartTile<N, Number>;
+  int const nx = t.nc[0], ny = t.nc[1], nz = t.nc[2];
+  LayerTiling l;
+  // a tile may run over the end of a row of tiles, except where the row's ends are neighbours
+  l.row_length = t.periodic[0] ? (nx + Tile::BX - 1) / Tile::BX * Tile::BX : nx;
+  l.tiles = (int)(((int64_t)((ny + Tile::BY - 1) / Tile::BY) * l.row_length + Tile::BX - 1) / Tile::BX);
+  // 2 to 8 layers per segment, of nearly equal length, with some 4000 workgroups where there are
+  // enough cells (longer segments leave the last round of workgroups uneven: 12 layers instead of 8
+  // cost 9% at FP64 k = 4 on 64^3 cells)
+  int const longest    = (int)std::max<int64_t>(2, std::min<int64_t>(8, (int64_t)nz * l.tiles / 4000));
+  l.segments           = (nz + longest - 1) / longest;
+  l.layers_per_segment = (nz + l.segments - 1) / l.segments;
+  return l;
+}
+
 // Whether the layered kernel is the faster one: where its fewer reads count, as src and dst outgrow
-// the 256 MB last-level cache, and with n <= 5 nodes per line, above which it has too few waves
-// (FP64 k = 5 on 48^3 cells 141 us against 131 single-layer, k = 7 on 40^3 207 against 183). The
-// line lies between, layered against single-layer in us: FP64 k = 4 50^3 cells (125 MB) 94 / 87,
-// 64^3 (262 MB) 165 / 177; k = 3 48^3 (57 MB) 44 / 43, 64^3 (134 MB) 85 / 94; k = 2 72^3 (81 MB)
-// 60 / 60, 88^3 (147 MB) 100 / 104. FP32 k = 4 56^3 (88 MB) 69 / 74, k = 3 64^3 (67 MB) 51 / 54,
-// k = 2 56^3 (19 MB) 21 / 23, k = 1 96^3 (28 MB) 30 / 34.
+// the 256 MB last-level cache, and with n <= 5 nodes per line, above which FP64 has too few waves
+// (k = 5 on 48^3 cells 141 us against 131 single-layer, k = 7 on 40^3 207 against 183; FP32 was not
+// tried there). The line lies between, layered against single-layer in us: FP64 k = 4 50^3 cells
+// (125 MB) 94 / 87, 64^3 (262 MB) 165 / 177; k = 3 48^3 (57 MB) 44 / 43, 64^3 (134 MB) 85 / 94; k = 2
+// 72^3 (81 MB) 60 / 60, 88^3 (147 MB) 100 / 104. FP32 k = 4 56^3 (88 MB) 69 / 74, k = 3 64^3 (67 MB)
+// 51 / 54, k = 2 56^3 (19 MB) 21 / 23, k = 1 96^3 (28 MB) 30 / 34.
+//
+// It also takes a box that fills the tiles: lanes without a cell cost as much as the others. Layered
+// against single-layer in us by the share of cells in the tiles: 1/50 (k = 1 on 1 x 1 x 480000)
+// 327 / 33, 1/8 (690 x 1 x 690) 52 / 20, 1/4 (k = 3 on 420 x 1 x 420) 106 / 66, 1/2 (k = 1 on
+// 350 x 4 x 350) 23 / 21, 0.6 (k = 4, 6 periodic cells along x) 161 / 134, 0.8 (8 along x) 143 / 135,
+// 0.82 (k = 1, 33 along x) 18.9 / 18.3, 0.9 and more 0.75 - 0.97 times. One layer alone leaves n = 2
+// with nothing to reuse (700 x 680 x 1 21.9 / 19.7; k = 2 on 400 x 400 x 1 20 / 21).
 template<int N, typename Number>
 bool use_layers(SipgArgs<Number> const & a)
 {
   int64_t const bytes = a.n_cells * (N * N * N * sizeof(Number));
-  return bytes >= 1000000 * (sizeof(Number) == 8 ? (N == 5 ? 180 : 90) : N >= 4 ? 60 : 15);
+  if(bytes < 1000000 * (sizeof(Number) == 8 ? (N == 5 ? 180 : 90) : N >= 4 ? 60 : 15))
+    return false;
+  int const     nz    = a.topo.nc[2];
+  int64_t const slots = (int64_t)layer_tiling<N, Number>(a.topo).tiles * CartTile<N, Number>::cells * nz;
+  return 20 * a.n_cells >= 17 * slots && (N > 2 || nz > 1);
 }
 
 template<int N, typename Number, ApplyMode mode>
 hipError_t launch_layers_n(SipgArgs<Number> a, hipStream_t stream)
 {
-  using Tile   = CartTile<N, Number>;
-  int const nx = a.topo.nc[0], ny = a.topo.nc[1], nz = a.topo.nc[2];
-  // a tile may run over the end of a row of tiles, except where the row's ends are neighbours
-  a.row_length = a.topo.periodic[0] ? (nx + Tile::BX - 1) / Tile::BX * Tile::BX : nx;
-  a.tiles = (int)(((int64_t)((ny + Tile::BY - 1) / Tile::BY) * a.row_length + Tile::BX - 1) / Tile::BX);
-  // 2 to 8 layers per segment, of nearly equal length, with some 4000 workgroups where there are
-  // enough cells (longer segments leave the last round of workgroups uneven: 12 layers instead of 8
-  // cost 9% at FP64 k = 4 on 64^3 cells)
-  int const longest    = (int)std::max<int64_t>(2, std::min<int64_t>(8, (int64_t)nz * a.tiles / 4000));
-  int const segments   = (nz + longest - 1) / longest;
-  a.layers_per_segment = (nz + segments - 1) / segments;
-  hipLaunchKernelGGL((sipg_cartesian_layers_kernel<N, Number, mode>), dim3((unsigned)a.tiles * segments),
-                     dim3(Tile::threads), (LdsLayout<N, Number>::bytes), stream, a);
+  LayerTiling const l  = layer_tiling<N, Number>(a.topo);
+  a.row_length         = l.row_length;
+  a.tiles              = l.tiles;
+  a.layers_per_segment = l.layers_per_segment;
+  hipLaunchKernelGGL((sipg_cartesian_layers_kernel<N, Number, mode>), dim3((unsigned)l.tiles * l.segments),
+                     dim3(CartTile<N, Number>::threads), (LdsLayout<N, Number>::bytes), stream, a);
   return hipGetLastError();
 }
 
@@ -1014,6 +1043,16 @@ std::vector<int> cartesian_line_map(int degree)
   }
 }
 
+template<typename Number>
+char const * cartesian_vmult_kernel(int degree, SipgArgs<Number> const & a)
+{
+  bool const layered = degree == 1 ? use_layers<2, Number>(a) : degree == 2 ? use_layers<3, Number>(a) :
+                       degree == 3 ? use_layers<4, Number>(a) : degree == 4 && use_layers<5, Number>(a);
+  return layered ? "sipg_cartesian_layers_kernel" : "sipg_cartesian_kernel";
+}
+
+template char const * cartesian_vmult_kernel<double>(int, SipgArgs<double> const &);
+template char const * cartesian_vmult_kernel<float>(int, SipgArgs<float> const &);
 template std::vector<int> cartesian_line_map<double>(int);
 template std::vector<int> cartesian_line_map<float>(int);
 

@@ -135,6 +135,10 @@ hipError_t launch_general_diagonal(Number * diag, double const * tab1d, SipgArgs
 template<typename Number>
 std::vector<int> cartesian_line_map(int degree);
 
+// The kernel that vmult and vmult_add launch for these arguments
+template<typename Number>
+char const * cartesian_vmult_kernel(int degree, SipgArgs<Number> const & args);
+
 template<typename Number>
 hipError_t launch_sipg_cartesian(int degree, ApplyMode mode, SipgArgs<Number> const & args,
                                  hipStream_t stream);

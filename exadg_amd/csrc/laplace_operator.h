@@ -34,6 +34,7 @@ public:
   virtual int64_t m() const                                                 = 0;
   virtual int64_t n_cells() const                                           = 0;
   virtual bool    is_affine() const                                         = 0;
+  virtual char const * vmult_kernel() const                                 = 0;
   virtual void    vmult(void * dst, void const * src, hipStream_t s) const     = 0;
   virtual void    vmult_add(void * dst, void const * src, hipStream_t s) const = 0;
   virtual void    calculate_diagonal(void * diag, hipStream_t s) const         = 0;
@@ -93,6 +94,11 @@ public:
   int64_t n() const { return m(); }
   int64_t n_cells() const override { return grid_->n_cells(); }
   bool    is_affine() const override { return grid_->affine(); }
+  char const * vmult_kernel() const override
+  {
+    return is_affine() ? cartesian_vmult_kernel<Number>(data_.degree, make_args(nullptr, nullptr, 0)) :
+                         "sipg_general_kernel";
+  }
 
   // OperatorBase::vmult / vmult_add / apply (operator_base.cpp:156-178, 264-310)
   void vmult(Number * dst, Number const * src, hipStream_t s) const;

@@ -90,6 +90,9 @@ int exadg_laplace_n_dofs(const exadg_laplace * op, int64_t * n_dofs);
 /* Number of cells, degree, precision, and whether the affine (Cartesian) kernel is used. */
 int exadg_laplace_info(const exadg_laplace * op, int64_t * n_cells, int * degree, int * precision,
                        int * is_affine);
+/* Diagnostics: the kernel that vmult and vmult_add launch for this operator (which one depends on
+ * the mesh, the degree and the precision); a static string. */
+int exadg_laplace_kernel(const exadg_laplace * op, const char ** name);
 
 /* OperatorBase::vmult(dst, src) (operator_base.h:175, operator_base.cpp:156-168 ->
  * apply :264-310): dst = A src for the homogeneous SIPG operator. dst is overwritten;

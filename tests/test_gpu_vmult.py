@@ -98,29 +98,47 @@ def test_fp32_rows_vanish_on_constants(k, torch_cuda, product):
 
 
 # affine meshes just above the sizes where the layered kernel takes over (15 and 60 MB a vector in
-# FP32, 90 MB in FP64): rows that end inside a tile, odd last rows of tiles, segments of unequal
-# length, a box shorter than a tile, one layer, and every periodic direction
+# FP32, 90 and 180 MB in FP64): rows that end inside a tile, odd last rows of tiles, segments of unequal
+# length, boxes shorter than a tile, one and two layers, and every periodic direction
 LAYERED = [
     (1, (79, 81, 75), "fp32", (0, 0, 0), (D, N, D, D, N, D)),
-    (1, (3, 7, 22500), "fp32", (0, 0, 0), (D,) * 6),
-    (1, (700, 680, 1), "fp32", (1, 1, 1), (D,) * 6),
+    (1, (3, 401, 395), "fp32", (0, 0, 0), (D,) * 6),
+    (1, (490, 481, 2), "fp32", (1, 1, 1), (D,) * 6),
+    (1, (113, 111, 113), "fp64", (0, 0, 0), (D, N, N, D, D, D)),
     (2, (53, 51, 53), "fp32", (1, 0, 0), (D, D, N, N, D, N)),
+    (2, (403, 397, 1), "fp32", (1, 1, 1), (D,) * 6),
     (3, (62, 61, 63), "fp32", (0, 1, 1), (N, D) * 3),
     (4, (49, 51, 50), "fp32", (1, 1, 0), (N,) * 6),
     (2, (76, 75, 74), "fp64", (0, 1, 0), (D, N, D, D, D, N)),
+    (3, (2, 300, 295), "fp64", (0, 0, 1), (D, D, N, D, D, D)),
+    (3, (58, 55, 57), "fp64", (1, 1, 0), (D, D, D, D, N, D)),
+    (4, (57, 58, 55), "fp64", (1, 0, 1), (D, D, N, D, D, N)),
+]
+# as long, but with tiles that they do not fill, or nothing to reuse: the single-layer kernel
+THIN = [
+    (1, (3, 7, 22500), "fp32", (0, 0, 0), (D,) * 6),
+    (1, (700, 680, 1), "fp32", (1, 1, 1), (D,) * 6),
+    (2, (1, 401, 400), "fp32", (1, 0, 0), (D,) * 6),
     (3, (2, 89, 1000), "fp64", (1, 0, 1), (D, D, N, D, D, D)),
+    (4, (1, 1, 121000), "fp32", (0, 0, 0), (D, N) * 3),
 ]
 
 
-@pytest.mark.parametrize("k,nc,prec,per,bc", LAYERED, ids=[f"k{c[0]}-{c[2]}-{c[1]}" for c in LAYERED])
-def test_layered_vmult_matches_oracle(k, nc, prec, per, bc, torch_cuda, product):
+@pytest.mark.parametrize("layered,row", [(True, c) for c in LAYERED] + [(False, c) for c in THIN],
+                         ids=[f"k{c[0]}-{c[2]}-{c[1]}" for c in LAYERED + THIN])
+def test_layered_vmult_matches_oracle(layered, row, torch_cuda, product):
     torch = torch_cuda
+    k, nc, prec, per, bc = row
     case = ("layered", k, nc, 0.0, (1.0, 1.1, 0.9), 0.0, 1, 1, per, bc)
     op_p, op_o = _build(product, case, product.FP32 if prec == "fp32" else product.FP64)
-    x = oracle.random_vector(op_o.n).astype(np.float32)
+    assert op_p.kernel == ("sipg_cartesian_layers_kernel" if layered else "sipg_cartesian_kernel")
+    x = oracle.random_vector(op_o.n)
+    if prec == "fp32":
+        x = x.astype(np.float32)
     y_ref = op_o.vmult(x.astype(np.float64))
     bar = 2e-6 if prec == "fp32" else 1e-12
-    xs = torch.from_numpy(x).cuda().to(op_p.dtype)
+    xs = torch.from_numpy(x).cuda()
+    assert xs.dtype == op_p.dtype
     ys = torch.full_like(xs, float("nan"))
     op_p.vmult(ys, xs)
     assert _rel(ys.cpu().numpy(), y_ref) <= bar
