@@ -169,6 +169,7 @@ def lib():
             "exadg_preconditioner_update": [vp, vp],
             "exadg_preconditioner_smooth": [vp, vp, vp, vp, vp],
             "exadg_preconditioner_destroy": [vp],
+            "exadg_preconditioner_mg_coarse_kernel": [vp, ctypes.POINTER(ctypes.c_char_p)],
             "exadg_preconditioner_mg_info": [vp, ip, ctypes.POINTER(ctypes.c_double), ip, ip],
             "exadg_preconditioner_mg_levels": [vp, ctypes.c_int, ip, ip, ip, ip, i64p],
             "exadg_cg_solve": [vp, vp, vp, vp, ctypes.POINTER(SolverData), ctypes.POINTER(SolveInfo),
@@ -424,6 +425,12 @@ class Preconditioner:
         n = (ctypes.c_int64 * 64)()
         check(lib().exadg_preconditioner_mg_levels(self._h, 64, ctypes.byref(nl), h, deg, dg, n))
         return [(h[i], deg[i], bool(dg[i]), n[i]) for i in range(nl.value)]
+
+    def mg_coarse_kernel(self):
+        """Name of what the coarse solve runs."""
+        name = ctypes.c_char_p()
+        check(lib().exadg_preconditioner_mg_coarse_kernel(self._h, ctypes.byref(name)))
+        return name.value.decode()
 
     def mg_info(self):
         nl = ctypes.c_int()

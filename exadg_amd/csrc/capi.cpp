@@ -495,6 +495,18 @@ int exadg_preconditioner_mg_info(const exadg_preconditioner * p, int * n_levels,
   });
 }
 
+int exadg_preconditioner_mg_coarse_kernel(const exadg_preconditioner * p, const char ** name)
+{
+  return guarded([&] {
+    require(p && name, "null argument");
+    require((p->kind & 0xff) == EXADG_PRECOND_MULTIGRID, "not a multigrid preconditioner");
+    if(p->kind & 0x100)
+      *name = static_cast<ExaDG::MultigridPreconditioner<float> const &>(*p->p).coarse_kernel();
+    else
+      *name = static_cast<ExaDG::MultigridPreconditioner<double> const &>(*p->p).coarse_kernel();
+  });
+}
+
 int exadg_preconditioner_mg_levels(const exadg_preconditioner * p, int max_levels, int * n_levels,
                                    int * h, int * degree, int * dg, int64_t * n)
 {

@@ -435,7 +435,7 @@ bool Q1Operator<Number>::chebyshev_step(Number * x_new, Number const * x, Number
 template<typename Number>
 bool Q1Operator<Number>::pcg(Q1PcgArgs<Number> args, hipStream_t s) const
 {
-  if(n_nodes_ > kQ1PcgMaxNodes)
+  if(!has_pcg())
     return false;
   args.W       = stencil_.data();
   args.q       = q_;

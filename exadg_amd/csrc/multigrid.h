@@ -196,6 +196,9 @@ public:
   // the coarse PCG solve in one launch (args without W, q and n); false if the level has no such form
   // or is too large for it
   virtual bool pcg(Q1PcgArgs<Number> /*args*/, hipStream_t /*s*/) const { return false; }
+  // what the coarse solves run on this level (diagnostics)
+  virtual char const * pcg_kernel() const { return "level_pcg"; }
+  virtual char const * chebyshev_kernel() const { return "chebyshev"; }
 };
 
 // continuous Q1 operator with strong Dirichlet constraints on the structured box
@@ -213,6 +216,11 @@ public:
                       Number const * dinv, Number f1, Number f2, bool has_old,
                       hipStream_t s) const override;
   bool pcg(Q1PcgArgs<Number> args, hipStream_t s) const override;
+  char const * pcg_kernel() const override { return has_pcg() ? "q1_pcg_kernel" : "level_pcg"; }
+  char const * chebyshev_kernel() const override
+  {
+    return classes_.size() ? "q1_chebyshev_kernel, node classes" : "q1_chebyshev_kernel, planes";
+  }
   Q1Topology const & q1_topology() const { return q_; }
   CGTopology const * cg_topology() const override { return &cg_; }
   std::vector<double> const & element_matrices() const { return mats_host_; }
@@ -220,6 +228,7 @@ public:
 private:
   // the stencil's rows by node class; empty if the nodes of a class differ
   std::vector<Number> stencil_classes(std::vector<double> const & W) const;
+  bool                has_pcg() const { return n_nodes_ <= kQ1PcgMaxNodes && stencil_.size() > 0; }
   Q1Weights<Number>   weights() const { return {stencil_.data(), classes_.data()}; }
 
   BoxTopology          topo_;
@@ -321,6 +330,11 @@ public:
   ChebyshevSmoother<Number> const & smoother(int l) const { return levels_[l].smoother; }
   ChebyshevSmoother<Number> const & coarse_chebyshev() const { return coarse_cheb_; }
   int                              last_coarse_iterations() const { return last_coarse_its_; }
+  char const *                     coarse_kernel() const
+  {
+    return data_.coarse_solver == CoarseSolver::chebyshev ? levels_[0].op->chebyshev_kernel() :
+                                                            levels_[0].op->pcg_kernel();
+  }
   // components for tests: transfer between level l-1 and l
   void prolongate_and_add(int l, Number * dst_fine, Number const * src_coarse, hipStream_t s) const;
   void restrict_and_add(int l, Number * dst_coarse, Number const * src_fine, hipStream_t s) const;

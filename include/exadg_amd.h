@@ -260,6 +260,9 @@ int exadg_preconditioner_destroy(exadg_preconditioner * p);
 int exadg_preconditioner_mg_info(const exadg_preconditioner * p, int * n_levels,
                                  double * lambda_max, int * chebyshev_degree,
                                  int * last_coarse_iterations);
+/* Diagnostics: what the coarse solve of a multigrid preconditioner runs (it depends on the coarse
+ * solver, the mesh and the precision); a static string. */
+int exadg_preconditioner_mg_coarse_kernel(const exadg_preconditioner * p, const char ** name);
 
 /* SolverData (solvers_and_preconditioners/solvers/solver_data.h:91-146) */
 typedef struct exadg_solver_data

@@ -75,7 +75,7 @@ def test_extrapolate(torch_cuda, product, order):
                                                     # the GEMM's tiles and split sums: one sample,
                                                     # unaligned rows (odd width), the smallest batch
                                                     # of the largest tile, one past a stage
-                                                    (1, 1, 7, 1), (2, 2, 33, 1025), (1, 4, 128, 16321),
+                                                    (1, 1, 7, 1), (1, 2, 1, 33), (2, 2, 33, 1025), (1, 4, 128, 16321),
                                                     (4, 3, 129, 2049)])
 def test_loss_and_grad_vs_oracle(torch_cuda, product, degree, history, width, B):
     torch = torch_cuda
