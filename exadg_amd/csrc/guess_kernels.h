@@ -24,7 +24,7 @@ struct FeatureScales
   float inv_t    = 1.f;
 };
 
-// C(i,j) = alpha sum_k A(i,k) B(k,j) (+ C if accumulate) (+ bias_j) (ReLU) (0 where mask(i,j) <= 0,
+// C(i,j) = sum_k A(i,k) B(k,j) (+ bias_j) (ReLU) (0 where mask(i,j) <= 0,
 // laid out as C), A(i,k) = A[i a_i + k a_k], B(k,j) = B[k b_k + j b_j], one of the two strides of
 // each being 1 (not a_i with b_k alone); row_sum (if not null) receives sum_k A(i,k). With a
 // workspace (gradients: sums over the batch) of >= s M (N + 1) floats the K range may be split over s
@@ -38,12 +38,10 @@ struct SgemmArgs
   int64_t       b_k, b_j;
   float *       C;
   int64_t       ldc;
-  float         alpha      = 1.f;
-  int           accumulate = 0;
-  float const * bias       = nullptr;
-  int           relu       = 0;
-  float const * mask       = nullptr;
-  float *       row_sum    = nullptr;
+  float const * bias    = nullptr;
+  int           relu    = 0;
+  float const * mask    = nullptr;
+  float *       row_sum = nullptr;
 };
 hipError_t launch_sgemm(SgemmArgs const & a, float * workspace, int64_t workspace_floats, hipStream_t s);
 template<typename In>

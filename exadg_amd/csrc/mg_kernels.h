@@ -64,11 +64,13 @@ hipError_t launch_q1_chebyshev(Number * x_new, Number const * x, Number const * 
                                Q1Topology const & q, Number f1, Number f2, bool has_old,
                                hipStream_t s);
 
-// PCG with point Jacobi on a Q1 level of at most kQ1PcgMaxNodes nodes, in one workgroup: x from zero to |r| <= max(1e-12, rel_tol |b|), with the mean of b and of every residual removed if
-// singular. r and v: n entries of workspace each; result: iterations, then 1 if a residual was not
+// PCG with point Jacobi on a Q1 level of at most kQ1PcgMaxNodes nodes, in one workgroup: x from zero
+// to |r| <= max(1e-12, rel_tol |b|), with the mean of b and of every residual removed if singular. r
+// and v: n entries of workspace each; result: iterations, then 1 if a residual was not
 // finite. The line lies where one workgroup's pass over the stencil takes as long as an iteration
-// driven from the host (whole solve, FP32 V-cycle, host-driven / here: 729 nodes 9.2 / 3.7 ms,
-// 1296 nodes 33 / 11.5 ms, 9261 nodes 21.8 / 15.6 ms, 17576 nodes 34.5 / 39.2 ms).
+// driven from the host, host-driven / here: whole solves with the FP32 V-cycle 729 nodes 9.2 / 3.7 ms,
+// 1296 nodes 33 / 11.5 ms, 9261 nodes 21.8 / 15.6 ms, 17576 nodes 34.5 / 39.2 ms; one V-cycle at 9261
+// nodes FP32 1401 / 999 us, FP64, which reads twice the bytes, 1441 / 1289 us.
 constexpr int kQ1PcgMaxNodes = 10000;
 template<typename Number>
 struct Q1PcgArgs

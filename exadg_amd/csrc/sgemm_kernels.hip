@@ -1,6 +1,6 @@
 // FP32 GEMM of the learned guess's network on the matrix cores, with strided operands.
 //
-//   C(i,j) = epilogue(alpha sum_k A(i,k) B(k,j)), A(i,k) = A[i a_i + k a_k], B(k,j) = B[k b_k + j b_j]
+//   C(i,j) = epilogue(sum_k A(i,k) B(k,j)), A(i,k) = A[i a_i + k a_k], B(k,j) = B[k b_k + j b_j]
 //
 // A workgroup of four waves computes a TM x TN tile, each wave a quadrant of (TM/32) x (TN/32)
 // blocks of v_mfma_f32_16x16x4f32 (FP32 operands and accumulation). Lane l supplies A(l%16, l/16)
@@ -93,9 +93,6 @@ struct Operand
 
 __device__ __forceinline__ float epilogue(SgemmArgs const & a, float v, int64_t i, int j)
 {
-  v *= a.alpha;
-  if(a.accumulate)
-    v += a.C[i * a.ldc + j];
   if(a.bias)
     v += a.bias[j];
   if(a.relu)

@@ -28,7 +28,7 @@ __device__ __forceinline__ void mat_apply(Table const M, Number const (&in)[N],
 }
 
 // out = A in for a centrosymmetric (Skew = false) or skew-centrosymmetric (Skew = true) A,
-// stored in even-odd form when Packed (see cs_packed / gen_packed), else as the plain row-major
+// stored in even-odd form when Packed (always in the Cartesian kernel, else see gen_packed), else as the plain row-major
 // matrix. Centro: out_i = E_i + O_i, out_{n-1-i} = E_i - O_i, middle output (odd n) from the
 // even part; skew: out_{n-1-i} = O_i - E_i and the middle output from the odd part.
 template<int N, bool Packed, bool Skew, typename Number, typename Table>
