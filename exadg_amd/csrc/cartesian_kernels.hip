@@ -27,10 +27,11 @@
 // registers and a longer start. What bounds them are LDS passes, vector instructions and the
 // vector-memory address unit together: FP64 k = 4 on 64^3 cells kept them busy for 76%, 60% and 73%
 // of the cycles (SQ_LDS_IDX_ACTIVE, SQ_ACTIVE_INST_VALU, TA_BUSY) when 41% of the LDS passes were
-// bank conflicts, hence strides and line assignments by bank and the shared even-odd parts. Medians
-// of one box, before / single-layer / layered: FP64 k = 4 on 64^3 cells 229 / 177 / 165 us (2.3 ->
-// 3.2 TB/s of src and dst); FP32 k = 6 on 31 x 45 x 27 49.0 / 46.4 us; FP64 k = 7 on 40^3
-// 262 / 183 us; FP32 k = 2 on 96^3 113 / 100 / 75 us.
+// bank conflicts, hence strides and line assignments by bank and the shared even-odd parts (now 58%
+// with 7% conflicts, 55% and 40%). Launches in turn in one process, before / single-layer / layered:
+// FP64 k = 4 on 64^3 cells 183 / 173 / 165 us (2.9 -> 3.2 TB/s of src and dst; 202 / - / 174 with
+// changing inputs), k = 3 on 64^3 90 / 86 / 77; FP32 k = 6 on 31 x 45 x 27 42.9 / 41.0; FP64 k = 7 on
+// 40^3 217 / 182; FP32 k = 2 on 96^3 95 / 91 / 68.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -93,9 +93,9 @@ __device__ __forceinline__ void source_line(Number const * __restrict__ src, int
 // normal-derivative vectors a = J^{-1} n of both sides, and the face tests added to the
 // Gauss-level residual before the transposed interpolation back to the nodes.
 //
-// What bounds it: the vector-memory address unit (busy 65 - 70% of the cycles), the vector
-// instructions (65% in FP32, 35% in FP64) and the LDS passes (55% / 47%), each waiting on the others
-// between barriers. x-neighbours of the workgroup's row are therefore read from LDS (their strided
+// What bounds it: LDS passes (busy 62% of the cycles in FP64 at k = 5, 66% in FP32 at k = 3), the
+// vector-memory address unit (52% / 31%) and the vector instructions (36% / 58%), each waiting on the
+// others between barriers; the address unit had been busy 65 - 70%. x-neighbours of the workgroup's row are therefore read from LDS (their strided
 // x-lines cost some 48 address cycles per load), the lanes' rows and columns of Dq come from LDS,
 // the face types and indices are 32-bit and the types taken once, and the LDS strides avoid bank
 // conflicts (GenLayout): FP64 k = 5 on 48^3 cells 651 -> 569 us (3.4 -> 3.9 TB/s of the 2.2 GB it

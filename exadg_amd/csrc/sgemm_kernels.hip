@@ -14,8 +14,8 @@
 // What bounds it: the matrix cores (157 TFLOP/s FP32) for the large batches, the length of one
 // tile's chain of stages for minibatches. The three products of a prediction (32768 x 128 x 500, x 128,
 // 32768 x 125 x 128, 6.3 GFLOP) take 104 us (61 TFLOP/s), 199 us with 64 x 64 tiles, one LDS buffer
-// and 4-byte loads; a gradient of 4096 samples with its eight products 182 us instead of 358, of
-// which 94 us are the products, 28 us the split sums (from 64 to 16 parts and fewer).
+// and 4-byte loads; a gradient of 4096 samples with its eight products 189 us instead of 358, of
+// which 100 us are the products, 30 us the split sums (from 64 to 16 parts and fewer).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
